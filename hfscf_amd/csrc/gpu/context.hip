@@ -20,6 +20,7 @@
 #include "misc.hpp"
 #include "noalloc.hpp"
 #include "private_segments.hpp"
+#include "rys.hpp"
 
 using namespace hfg;
 
@@ -45,23 +46,25 @@ hipStream_t shared_scratch_stream(int device) {
     return streams[device];
 }
 
-// Streams and launch order of the class launches (J/K, or the gradient when grad): the classes
+// Streams and launch order of the class launches (J/K, or the gradient of a precision when grad): the classes
 // of the shared stream (on_shared_stream) run there (-1); the others are balanced over the side
 // streams, onto the least loaded one, by the weights w (the FLOP model at set-up, the measured
 // kernel times after autotuning). The launch order is the cooperative-kernel classes first (one
 // quartet per workgroup at a time: few workgroups on long serial chains, whose latency then
 // hides under the wide launches instead of trailing the build), then heaviest first.
-void assign_streams(hfg_ctx* c, bool grad, const std::vector<double>& w) {
-    std::vector<int>& map = grad ? c->grad_stream : c->class_stream;
+void assign_streams(hfg_ctx* c, bool grad, bool mixed, const std::vector<double>& w) {
+    std::vector<int>& map = grad ? c->grad_stream[mixed ? 1 : 0] : c->class_stream;
     map.assign(c->classes.size(), 0);
     std::vector<size_t> ord(c->classes.size());
     std::iota(ord.begin(), ord.end(), 0);
-    auto coop = [&](size_t k) { return grad ? c->classes[k].gcoop : c->classes[k].coop; };
+    auto coop = [&](size_t k) {
+        return grad ? c->classes[k].gcoop && !grad_on_rys(c, c->classes[k], mixed) : c->classes[k].coop;
+    };
     std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) {
         if (coop(x) != coop(y)) return coop(x);
         return w[x] > w[y];
     });
-    std::vector<int>& order = grad ? c->grad_order : c->class_order;
+    std::vector<int>& order = grad ? c->grad_order[mixed ? 1 : 0] : c->class_order;
     order.assign(ord.begin(), ord.end());
     // the balance is over hardware queues: side streams on one queue count as one, the first of
     // them takes the queue's classes, and a queue shared with the shared stream starts with the
@@ -72,11 +75,11 @@ void assign_streams(hfg_ctx* c, bool grad, const std::vector<double>& w) {
     for (int s = 0; s < nside; ++s) rep[s] = c->side_queue[s] == s;
     for (size_t k = 0; k < c->classes.size(); ++k) {
         const ClassWork& cw = c->classes[k];
-        if (on_shared_stream(c, cw, grad) && c->heavy_queue >= 0) load[c->heavy_queue] += w[k];
+        if (on_shared_stream(c, cw, grad, mixed) && c->heavy_queue >= 0) load[c->heavy_queue] += w[k];
     }
     for (size_t k : ord) {
         const ClassWork& cw = c->classes[k];
-        if (on_shared_stream(c, cw, grad)) {
+        if (on_shared_stream(c, cw, grad, mixed)) {
             map[k] = -1;
             continue;
         }
@@ -904,8 +907,8 @@ int setup_geometry(hfg_ctx* c) {
             wj.push_back(cw.jk_flops());
             wg.push_back(cw.grad_flops);
         }
-        assign_streams(c, false, wj);
-        assign_streams(c, true, wg);
+        assign_streams(c, false, false, wj);
+        for (bool mixed : {false, true}) assign_streams(c, true, mixed, wg);
     }
     // gather lists (one output tile per block pair) and per-molecule item lists
     std::vector<std::vector<GatherEntry>> lj(nbp), lk(nbp);
@@ -1010,6 +1013,31 @@ int setup_geometry(hfg_ctx* c) {
             ao[s] = c->pure ? c->pure_off[s] : c->cart_off[s];
             nf[s] = nfun(c->L[s], c->pure);
         }
+        HFG_CHECK(c, c->d_cart_off.upload(c->cart_off, c->stream));
+        // Cartesian functions as sums of output functions, for the Cartesian densities
+        std::vector<MolCart> mc;
+        std::vector<CartTerms> terms;
+        c->nc_total = 0;
+        c->max_ncart = 0;
+        for (const auto& M : c->mols) {
+            mc.push_back(MolCart{c->pure ? (long long)c->nc_total : M.moff, M.ncart, (int)terms.size()});
+            c->nc_total += (size_t)M.ncart * M.ncart;
+            c->max_ncart = std::max(c->max_ncart, M.ncart);
+            if (!c->pure) continue;
+            std::vector<CartTerms> t(M.ncart, CartTerms{});
+            for (int s = M.shell0; s < M.shell0 + M.nshell; ++s)
+                for (int k = 0; k < nfun(c->L[s], true); ++k) {
+                    const SphTerms st = sph_terms(c->L[s], k);
+                    for (int x = 0; x < st.n; ++x) {
+                        CartTerms& ct = t[c->cart_off[s] + st.c[x]];
+                        ct.f[ct.n] = c->pure_off[s] + k;
+                        ct.w[ct.n++] = st.w[x];
+                    }
+                }
+            terms.insert(terms.end(), t.begin(), t.end());
+        }
+        HFG_CHECK(c, c->d_mol_cart.upload(mc, c->stream));
+        HFG_CHECK(c, c->d_cart_terms.upload(terms, c->stream));
         HFG_CHECK(c, c->d_shell_ao.upload(ao, c->stream));
         HFG_CHECK(c, c->d_shell_nf.upload(nf, c->stream));
         HFG_CHECK(c, c->d_shell_mol.upload(c->shell_mol, c->stream));
@@ -1311,7 +1339,8 @@ hipError_t hfg::launch_jk_class(hfg_ctx* c, const ClassWork& cw, const JkArgs& a
 int hfg::check_private_segments(hfg_ctx* c, bool grad) {
     const bool mixed = c->opt.precision == HFG_MIXED;
     for (const ClassWork& cw : c->classes) {
-        if (grad ? cw.gcoop : cw.coop) continue;  // the cooperative kernels hold their tables in LDS
+        // the cooperative and Rys kernels hold their tables in LDS
+        if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop) continue;
         if ((grad ? grad_uses_coop(cw.la, cw.lb, cw.lc, cw.ld) : jk_uses_coop(cw.la, cw.lb, cw.lc, cw.ld)))
             return fail(c, HFG_ERR_UNSUPPORTED, "the class needs the cooperative kernel, whose LDS does not fit a "
                                                 "workgroup on this device");
@@ -1367,7 +1396,8 @@ int hfg_create(hfg_ctx** out, int device, const hfg_options* opt) {
     }
     if (hipDeviceGetAttribute(&c->max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
         c->max_lds = 65536;
-    if (noalloc_scratch(device, &c->scratch) != hipSuccess) {  // hfg_build_jk_noalloc's fixed scratch
+    // hfg_build_jk_noalloc's fixed scratch, the Rys tables
+    if (noalloc_scratch(device, &c->scratch) != hipSuccess || rys_table(device, &c->rys) != hipSuccess) {
         hfg_destroy(c);
         return HFG_ERR_HIP;
     }
@@ -1632,8 +1662,10 @@ int hfg_autotune(hfg_ctx* c, int what) {
         for (size_t k = 0; k < c->classes.size(); ++k) {
             ClassWork& cw = c->classes[k];
             bool& use_coop = grad ? cw.gcoop : cw.coop;
-            const bool coop_ok = grad ? cw.gcoop_ok : cw.coop_ok;
-            const bool reg_ok = cw.la + cw.lb + cw.lc + cw.ld < kCoopRequiredL;
+            // a class on the Rys gradient kernel only has its grid to choose (fixed workgroup size)
+            const bool rys = grad && grad_on_rys(c, cw, c->opt.precision == HFG_MIXED);
+            const bool coop_ok = !rys && (grad ? cw.gcoop_ok : cw.coop_ok);
+            const bool reg_ok = !rys && cw.la + cw.lb + cw.lc + cw.ld < kCoopRequiredL;
             LaunchShape& shape = grad ? cw.grad_shape : cw.jk_shape;
             bool best_coop = use_coop;
             LaunchShape best = shape;
@@ -1658,6 +1690,9 @@ int hfg_autotune(hfg_ctx* c, int what) {
                 for (int b : blocks)
                     for (int g : grids)
                         if ((r = trial(false, LaunchShape{g, b}))) return r;
+            if (rys)
+                for (int g : grids)
+                    if ((r = trial(use_coop, LaunchShape{g, 256}))) return r;
             if (coop_ok && (!reg_ok || cw.la + cw.lb + cw.lc + cw.ld >= kCoopTrialMinL))
                 for (int g : grids)
                     if ((r = trial(true, LaunchShape{g, 0}))) return r;
@@ -1666,7 +1701,7 @@ int hfg_autotune(hfg_ctx* c, int what) {
             measured[k] = best_ms;
         }
         // rebalance the side streams on the measured times of the chosen shapes
-        assign_streams(c, kind == 2, measured);
+        assign_streams(c, grad, c->opt.precision == HFG_MIXED, measured);
     }
     return HFG_OK;
 }
@@ -1927,6 +1962,10 @@ void hfg_destroy(hfg_ctx* c) {
     c->d_goff.release();
     c->d_gcnt.release();
     c->d_gc_p0.release();
+    c->d_Dc.release();
+    c->d_cart_off.release();
+    c->d_mol_cart.release();
+    c->d_cart_terms.release();
     c->d_one_sh.release();
     c->d_eri_out.release();
     c->d_one_pairs.release();

@@ -15,6 +15,7 @@
 #include "launch_bounds.hpp"
 #include "oneint.hpp"
 #include "private_segments.hpp"
+#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -143,8 +144,8 @@ struct hfg_ctx {
     hipStream_t heavy = nullptr;
     hipEvent_t ev_heavy_join = nullptr;
     std::vector<int> class_stream;  // side stream of each class's J/K launch (-1: the shared stream)
-    std::vector<int> grad_stream;   // the same for the gradient launches
-    std::vector<int> class_order, grad_order;  // launch order of the classes (J/K, gradient)
+    std::vector<int> grad_stream[2];  // the same for the gradient launches, FP64 and mixed
+    std::vector<int> class_order, grad_order[2];  // launch order of the classes (J/K, gradient)
     // hardware queue of each side stream and of the shared stream (equal values: one queue, whose
     // kernels run one after another); the stream balance spreads the classes over the queues
     int side_queue[hfg::kSideStreams] = {};
@@ -226,6 +227,14 @@ struct hfg_ctx {
     DevBuf<double> d_one_alpha, d_one_coef, d_one_xyz, d_one_Z, d_one_buf;
     DevBuf<int> d_hess_cart;  // first Cartesian function per shell (hfg_hessian_2e)
     DevBuf<int4> d_hess_items;  // its work items (hfg::HItem, four ints)
+    // the Cartesian densities of the Rys gradient kernels (rys_grad.hpp)
+    const double* rys = nullptr;  // the device's quadrature tables
+    int max_ncart = 0;            // largest molecule's Cartesian function count
+    size_t nc_total = 0;          // sum of their squares
+    DevBuf<double> d_Dc;
+    DevBuf<int> d_cart_off;  // global shell -> first Cartesian function in its molecule
+    DevBuf<hfg::MolCart> d_mol_cart;
+    DevBuf<hfg::CartTerms> d_cart_terms;
     // launch graphs of the J/K build (keyed by precision and density screening)
     std::vector<hfg::JkGraph> graphs;
     bool class_timed = false;  // the last J/K build bracketed each class launch with events
@@ -263,10 +272,15 @@ namespace hfg {
 // a J/K build that is captured in a graph), or only those on the shared stream.
 enum class ClassSet { All, Side, Shared };
 
+// Streams of the class launches (J/K, or the gradient in the context's precision when grad).
+inline const std::vector<int>& class_streams(const hfg_ctx* c, bool grad) {
+    return grad ? c->grad_stream[c->opt.precision == HFG_MIXED ? 1 : 0] : c->class_stream;
+}
+
 // Number of classes that run on the shared stream (J/K, or the gradient when grad). Their
 // device-queue counters come first ([0, n)), the side-stream classes' after them.
 inline int shared_class_count(const hfg_ctx* c, bool grad) {
-    const std::vector<int>& streams = grad ? c->grad_stream : c->class_stream;
+    const std::vector<int>& streams = class_streams(c, grad);
     return (int)std::count(streams.begin(), streams.end(), -1);
 }
 
@@ -277,7 +291,7 @@ inline int shared_class_count(const hfg_ctx* c, bool grad) {
 template <typename F>
 inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn, bool grad = false,
                                             ClassSet set = ClassSet::All, bool join_shared = true) {
-    const std::vector<int>& streams = grad ? c->grad_stream : c->class_stream;
+    const std::vector<int>& streams = class_streams(c, grad);
     const bool side = set != ClassSet::Shared, shared = set != ClassSet::Side;
     hipError_t e = hipEventRecord(c->ev_fork, main);
     if (e != hipSuccess) return e;
@@ -287,7 +301,7 @@ inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn
     if (shared && (e = hipStreamWaitEvent(c->heavy, c->ev_fork, 0)) != hipSuccess) return e;
     // the shared-stream classes first: they are few workgroups of long latency, and launched
     // after the side streams' persistent grids they would wait for compute units to drain
-    const std::vector<int>& order = grad ? c->grad_order : c->class_order;
+    const std::vector<int>& order = grad ? c->grad_order[c->opt.precision == HFG_MIXED ? 1 : 0] : c->class_order;
     int q = 0;
     for (int pass = 0; pass < 2; ++pass)
         for (size_t n = 0; n < c->classes.size(); ++n) {
@@ -315,25 +329,33 @@ inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn
 // there in every build.
 constexpr int kGradConcurrentBytes = 4096;
 
+// Whether the FP64 gradient of a class runs the Rys kernel (rys_grad.hpp): from L = 4, where the
+// register kernels spill (2.7 KB per lane at (pp|pp) to 13 KB at (dd|pp), all slower: (pp|pp) of
+// (H2O)16 44 ms against 28, of water 2.8 ms against 0.06) and the program kernel, from L = 7, works
+// on one primitive quartet at a time; a context that asks for the program kernels (coop_min_l)
+// keeps them.
+inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
+    const int l = cw.la + cw.lb + cw.lc + cw.ld;
+    return !mixed && l >= kRysGradMinL && (c->opt.coop_min_l == 0 || l < c->opt.coop_min_l);
+}
+
 // Whether a class launch runs on the device's shared stream (one kernel at a time): J/K register
 // kernels whose scratch bound is above kJkSharedBytes; gradient register kernels whose private
-// segment in this build (the larger of the FP64 and mixed kernels) is above kGradConcurrentBytes
-// (the scratch bound decides where the table has no entry).
-inline bool on_shared_stream(const hfg_ctx* c, const ClassWork& cw, bool grad) {
-    if (grad ? cw.gcoop : cw.coop) return false;
+// segment in this build is above kGradConcurrentBytes (the scratch bound decides where the table
+// has no entry).
+inline bool on_shared_stream(const hfg_ctx* c, const ClassWork& cw, bool grad, bool mixed) {
+    if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop) return false;
     if (!grad) return class_spills(cw.la, cw.lb, cw.lc, cw.ld, false);
-    const int b64 = private_segment_bytes(true, false, cw.la, cw.lb, cw.lc, cw.ld, c->pure);
-    const int b32 = private_segment_bytes(true, true, cw.la, cw.lb, cw.lc, cw.ld, c->pure);
-    if (b64 < 0 || b32 < 0) return class_spills(cw.la, cw.lb, cw.lc, cw.ld, true);
-    return std::max(b64, b32) > kGradConcurrentBytes;
+    const int b = private_segment_bytes(true, mixed, cw.la, cw.lb, cw.lc, cw.ld, c->pure);
+    return b < 0 ? class_spills(cw.la, cw.lb, cw.lc, cw.ld, true) : b > kGradConcurrentBytes;
 }
 
 // Stream of a class launch (J/K or gradient): a kernel of the shared stream always runs there,
 // also while autotuning tries it for a class that is on a side stream.
 inline hipStream_t class_launch_stream(hfg_ctx* c, size_t k, bool grad) {
     const ClassWork& cw = c->classes[k];
-    const int s = (grad ? c->grad_stream : c->class_stream)[k];
-    if (s < 0 || on_shared_stream(c, cw, grad)) return c->heavy;
+    const int s = class_streams(c, grad)[k];
+    if (s < 0 || on_shared_stream(c, cw, grad, c->opt.precision == HFG_MIXED)) return c->heavy;
     return c->side[s];
 }
 

@@ -1,6 +1,7 @@
 // Run-time dispatch of the adjoint gradient kernels and the fixed-order slab reduction.
 #include "coop_grad.hpp"
 #include "launch_bounds.hpp"
+#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -16,17 +17,16 @@ HFG_FOR_CLASSES(HFG_DECL)
 
 namespace {
 
-// The register kernels (FP64 or FP32) of the classes below L = 7; the classes from L = 7 up run
-// the cooperative kernel (coop_grad.hpp), launched by the context, and have no register kernel.
+// The register kernels: FP64 below L = kRysGradMinL (from there the context launches the Rys
+// kernel), mixed below L = 7 (from there it launches the cooperative kernel, coop_grad.hpp).
 template <int A, int B, int C, int D, bool P>
 hipError_t grad_class(const GradArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
-    if constexpr (grad_uses_coop(A, B, C, D)) {
-        return hipErrorInvalidValue;
-    } else {
-        const LaunchShape bs = scratch_safe_shape(A, B, C, D, true, sh, nitems);
-        return mixed ? launch_grad_class32<A, B, C, D, P>(a, nitems, bs, s)
-                     : launch_grad_class64<A, B, C, D, P>(a, nitems, bs, s);
-    }
+    const LaunchShape bs = scratch_safe_shape(A, B, C, D, true, sh, nitems);
+    if constexpr (!grad_uses_coop(A, B, C, D))
+        if (mixed) return launch_grad_class32<A, B, C, D, P>(a, nitems, bs, s);
+    if constexpr (A + B + C + D < kRysGradMinL)
+        if (!mixed) return launch_grad_class64<A, B, C, D, P>(a, nitems, bs, s);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace

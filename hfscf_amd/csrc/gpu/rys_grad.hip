@@ -1,0 +1,49 @@
+// Run-time dispatch of the Rys gradient kernels and the Cartesian densities that they read.
+#include "rys_grad.hpp"
+
+namespace hfg {
+
+#define HFG_RYS_CASE(A, B, C, D)                                                                  \
+    if constexpr (A + B + C + D >= kRysGradMinL)                                                  \
+        if (la == A && lb == B && lc == C && ld == D) return launch_rys_grad_class<A, B, C, D>(b, sh, s);
+
+#define HFG_DECL(A, B, C, D) \
+    template <>              \
+    hipError_t launch_rys_grad_class<A, B, C, D>(const RysGradArgs&, LaunchShape, hipStream_t);
+HFG_FOR_CLASSES(HFG_DECL)
+#undef HFG_DECL
+
+hipError_t launch_rys_grad(int la, int lb, int lc, int ld, const RysGradArgs& a, int nitems, LaunchShape sh,
+                           hipStream_t s) {
+    if (nitems == 0) return hipSuccess;
+    RysGradArgs b = a;
+    b.g.nitems = nitems;
+    HFG_FOR_CLASSES(HFG_RYS_CASE)
+    return hipErrorInvalidValue;
+}
+
+// One thread per Cartesian element; 2 x 2 terms at most, so it moves little more than D and Dc.
+__global__ __launch_bounds__(256) void to_cart_kernel(const double* __restrict__ D, const MolDev* __restrict__ mols,
+                                                      const MolCart* __restrict__ mc, const CartTerms* __restrict__ terms,
+                                                      double* __restrict__ Dc) {
+    const MolCart m = mc[blockIdx.y];
+    const MolDev md = mols[blockIdx.y];
+    const double* Dm = D + md.moff;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < m.n * m.n; e += gridDim.x * 256) {
+        const int i = e / m.n, j = e - i * m.n;
+        const CartTerms ti = terms[m.row0 + i], tj = terms[m.row0 + j];
+        double v = 0.0;
+        for (int x = 0; x < ti.n; ++x)
+            for (int y = 0; y < tj.n; ++y) v += ti.w[x] * tj.w[y] * Dm[(size_t)ti.f[x] * md.n + tj.f[y]];
+        Dc[m.off + e] = v;
+    }
+}
+
+hipError_t launch_to_cart(const double* D, const MolDev* mols, const MolCart* mc, int nmol, int max_ncart,
+                          const CartTerms* terms, double* Dc, hipStream_t s) {
+    const int grid = std::max(1, std::min(1024, (max_ncart * max_ncart + 255) / 256));
+    hipLaunchKernelGGL(to_cart_kernel, dim3(grid, nmol), dim3(256), 0, s, D, mols, mc, terms, Dc);
+    return hipGetLastError();
+}
+
+}  // namespace hfg
