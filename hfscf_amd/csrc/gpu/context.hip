@@ -400,6 +400,7 @@ int setup_geometry(hfg_ctx* c) {
     // before them; the storage keeps all of them.
     double mq = 0.0;
     for (size_t k = 0; k < pp0.size(); ++k) mq = std::max(mq, std::fabs(pp1[k].w) / std::sqrt(pp0[k].x));
+    c->prim_mq = mq;
     const double sig_cut = std::min(1e-16, c->opt.integral_tol / 1e4);
     {
         const double cut = sig_cut;
@@ -1974,8 +1975,10 @@ void hfg_destroy(hfg_ctx* c) {
     c->d_one_xyz.release();
     c->d_one_Z.release();
     c->d_one_buf.release();
-    c->d_hess_cart.release();
-    c->d_hess_items.release();
+    c->d_hess_pairs.release();
+    c->d_hess_prims.release();
+    c->d_hess_segs.release();
+    c->d_hess_queue.release();
     c->d_gc_p1.release();
     c->d_gc_K.release();
     c->d_gJ_off.release();

@@ -15,6 +15,7 @@
 #include "launch_bounds.hpp"
 #include "oneint.hpp"
 #include "private_segments.hpp"
+#include "rys_hess.hpp"
 #include "rys_layout.hpp"
 
 namespace hfg {
@@ -185,6 +186,7 @@ struct hfg_ctx {
     std::vector<double> gkey;
     std::vector<int> goff, gcnt;
     std::vector<int> gc_nfull;  // primitive pairs stored per group pair of each list
+    double prim_mq = 0.0;   // largest |K| / sqrt(p) of a primitive pair (bounds |K_cd| / sqrt(p + q))
     double tol = 0.0;       // quartets with psmean_ab psmean_cd below this are skipped
     double elem_tol = 0.0;  // hfscf's element screen and Cartesian diagonal (0 without screening)
     // work
@@ -225,8 +227,11 @@ struct hfg_ctx {
     DevBuf<hfg::OneShell> d_one_sh;
     DevBuf<int2> d_one_pairs;
     DevBuf<double> d_one_alpha, d_one_coef, d_one_xyz, d_one_Z, d_one_buf;
-    DevBuf<int> d_hess_cart;  // first Cartesian function per shell (hfg_hessian_2e)
-    DevBuf<int4> d_hess_items;  // its work items (hfg::HItem, four ints)
+    // hfg_hessian_2e: shell pairs, their primitive pairs, the classes' work-item segments and queues
+    DevBuf<hfg::HessPair> d_hess_pairs;
+    DevBuf<double4> d_hess_prims;
+    DevBuf<hfg::HessSegment> d_hess_segs;
+    DevBuf<unsigned long long> d_hess_queue;
     // the Cartesian densities of the Rys gradient kernels (rys_grad.hpp)
     const double* rys = nullptr;  // the device's quadrature tables
     int max_ncart = 0;            // largest molecule's Cartesian function count
