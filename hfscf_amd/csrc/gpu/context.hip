@@ -1970,6 +1970,7 @@ void hfg_destroy(hfg_ctx* c) {
     c->d_one_sh.release();
     c->d_eri_out.release();
     c->d_one_pairs.release();
+    c->d_one_terms.release();
     c->d_one_alpha.release();
     c->d_one_coef.release();
     c->d_one_xyz.release();

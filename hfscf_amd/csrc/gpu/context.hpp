@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../../include/hfgpu.h"
+#include "coop.hpp"
 #include "coop_args.hpp"
 #include "gather.hpp"
 #include "gc.hpp"
@@ -226,6 +227,7 @@ struct hfg_ctx {
     // one-electron integrals (hfg_oneint, hfg_oneint_gradient)
     DevBuf<hfg::OneShell> d_one_sh;
     DevBuf<int2> d_one_pairs;
+    DevBuf<hfg::SphTerms> d_one_terms;  // output functions as sums of Cartesian functions
     DevBuf<double> d_one_alpha, d_one_coef, d_one_xyz, d_one_Z, d_one_buf;
     // hfg_hessian_2e: shell pairs, their primitive pairs, the classes' work-item segments and queues
     DevBuf<hfg::HessPair> d_hess_pairs;

@@ -2,429 +2,495 @@
 // molecule, and their first-derivative contractions for the RHF gradient. They replace what hfscf
 // computes on the CPU in OSOverlap, OSKinetic and OSNuclear and their first derivatives (hfscf:
 // src/integrals/hfscf_osoverlap.cpp:10, hfscf_osnuclear.cpp:17-83, hfscf_osoverlapderiv1.cpp:8,
-// hfscf_oskineticderiv1.cpp:8, hfscf_osnuclearderiv1.cpp:15), with McMurchie-Davidson Hermite
-// expansions: S and T from the 1-D Hermite coefficients E^{ij}_0, V from E^{ij}_t and the Hermite
-// Coulomb integrals R_tuv (Boys values from the device table), derivatives by the shifts
+// hfscf_oskineticderiv1.cpp:8, hfscf_osnuclearderiv1.cpp:15): S and T from the 1-D overlap
+// recursion, V from the McMurchie-Davidson Hermite coefficients E^{ij}_t and the Hermite Coulomb
+// integrals R_tuv (Boys values from the device table), derivatives by the shifts
 // d/dA_x |a> = 2 alpha |a + 1_x> - a_x |a - 1_x>.
 //
-// One lane per shell pair for S and T, per shell pair and nucleus for V (added into V with
-// atomics), and per ordered shell pair and part (the overlap and kinetic terms, or one nucleus)
-// for the gradient terms; angular momenta up to 2, so the derivative shifts reach 3 on the bra and,
-// for T, 5 on the ket. This is O(N^2 natom) work next to the O(N^4) two-electron build, so the
-// kernels keep their tables in per-lane arrays sized for the largest shells rather than
-// specialising per class.
+// One kernel per pair class (la lb), everything unrolled so that the tables are registers. Sixteen
+// lanes take a shell pair; a lane's item is a primitive pair and a slice of the nuclei. The sum
+// over nuclei is taken in the Hermite basis, V_ab = sum_tuv E^{ab}_tuv (sum_C -Z_C R_tuv(P - C)), so
+// a nucleus costs its R_tuv and one multiply-add per tuv, and the expansion to the components
+// happens once per item. In the gradient the same Hermite sums give the derivatives with respect to
+// A and to P (A and B together), and a nucleus's own derivative is one more contraction of R with
+// the primitive pair's Hermite density. All blocks are Cartesian; the spherical basis enters by
+// one transformation of the matrices (densities before, integrals after).
+//
+// Bound: FP64 VALU of R_tuv (the Boys step and the recursion). Measured per call, with the host's
+// copies: (H2O)16 / cc-pVDZ S, T, V 0.54 ms (3.2 with one lane per pair and nucleus on tables in
+// scratch); (H2O)8 / cc-pVDZ gradient terms 0.27 ms
+// (7.9).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <vector>
 
 #include "boys.hpp"
+#include "cart.hpp"
 #include "context.hpp"
 #include "coop.hpp"
 #include "oneint.hpp"
+#include "rys_grad.hpp"
 
 namespace hfg {
 
 namespace {
 
-constexpr int kOneMaxL = 2;                   // largest shell angular momentum
-constexpr int kRN = 2 * kOneMaxL + 1;         // largest total order of R_tuv (gradient)
-constexpr int kRSize = (kRN + 1) * (kRN + 2) * (kRN + 3) / 6;  // R_tuv with t + u + v <= kRN
+constexpr int kOneLanes = 16;   // lanes per shell pair
+constexpr int kOneBlock = 64;   // threads per workgroup: four shell pairs
+constexpr int kOneLdsAtoms = 1024;  // gradient sums of up to this many nuclei in LDS
+// A primitive pair with exp(-ab/p |AB|^2) c_a c_b below this adds nothing to a double (the integrals
+// are at most a few hundred times it): about half of a water cluster's primitive pairs.
+constexpr double kOneTiny = 1e-40;
 
-// Cartesian exponents of component k of a shell of angular momentum L (hfscf's order: xx, xy, xz,
-// yy, yz, zz; hfscf: src/integrals/hfscf_shell.cpp:27-40).
-__device__ inline void cart_lmn(int L, int k, int* l) {
-    int n = 0;
-    for (int i = 0; i <= L; ++i)
-        for (int j = 0; j <= i; ++j, ++n)
-            if (n == k) {
-                l[0] = L - i;
-                l[1] = i - j;
-                l[2] = j;
-                return;
-            }
-}
-
-__device__ inline int ncart1(int L) { return (L + 1) * (L + 2) / 2; }
-
-// Hermite expansion coefficients E^{ij}_t of one direction, i < ni <= EI, j < nj <= EJ: the
-// integrals need EI = Lmax + 1, EJ = Lmax + 3 (kinetic: ket + 2), the gradient one more of each.
-template <int EI, int EJ>
-struct Herm1 {
-    static constexpr int kEj = EJ, kEt = EI + EJ - 1;  // t <= i + j
-    double e[EI * EJ * kEt];
-    int ni, nj;
-    __device__ double get(int i, int j, int t) const {
-        if (i < 0 || j < 0 || t < 0 || t > i + j || i >= ni || j >= nj) return 0.0;
-        return e[(i * kEj + j) * kEt + t];
-    }
-    __device__ void build(int imax, int jmax, double p, double xpa, double xpb) {
-        ni = imax + 1;
-        nj = jmax + 1;
-        const double o2p = 0.5 / p;
-        for (int i = 0; i <= imax; ++i)
-            for (int j = 0; j <= jmax; ++j)
-                for (int t = 0; t <= i + j; ++t) {
-                    double v;
-                    if (i == 0 && j == 0)
-                        v = 1.0;
-                    else if (i > 0)
-                        v = o2p * get_partial(i - 1, j, t - 1) + xpa * get_partial(i - 1, j, t) +
-                            (t + 1) * get_partial(i - 1, j, t + 1);
-                    else
-                        v = o2p * get_partial(i, j - 1, t - 1) + xpb * get_partial(i, j - 1, t) +
-                            (t + 1) * get_partial(i, j - 1, t + 1);
-                    e[(i * kEj + j) * kEt + t] = v;
-                }
-    }
-    // entries already built (the recursion reads only lower i, or lower j at i = 0)
-    __device__ double get_partial(int i, int j, int t) const {
-        if (t < 0 || t > i + j) return 0.0;
-        return e[(i * kEj + j) * kEt + t];
-    }
-};
-
-__device__ inline int ridx(int t, int u, int v) {
+HFG_HD int rsize(int n) { return (n + 1) * (n + 2) * (n + 3) / 6; }
+HFG_HD int ridx(int t, int u, int v) {
     const int s = t + u + v;
     return s * (s + 1) * (s + 2) / 6 + (s - t) * (s - t + 1) / 2 + v;
 }
 
-// Boys values F_0..F_N(T) scaled by `scale`, N <= kRN, from the device table.
-__device__ inline void boys_n(int N, double T, const double* tab, double* F) {
-    switch (N) {
-        case 0: boys_eval<0, double>(T, tab, 1.0, F); break;
-        case 1: boys_eval<1, double>(T, tab, 1.0, F); break;
-        case 2: boys_eval<2, double>(T, tab, 1.0, F); break;
-        case 3: boys_eval<3, double>(T, tab, 1.0, F); break;
-        case 4: boys_eval<4, double>(T, tab, 1.0, F); break;
-        default: boys_eval<kRN, double>(T, tab, 1.0, F); break;
-    }
-}
-
-// Hermite Coulomb integrals R_tuv(p, PC), t + u + v <= N, by the recursion over the auxiliary
-// order from R^(m)_000 = (-2p)^m F_m(p |PC|^2), one order at a time.
-__device__ inline void hermite_r(int N, double p, const double* pc, const double* tab, double* R) {
-    double F[kRN + 1];
-    boys_n(N, p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]), tab, F);
-    double prev[kRSize], cur[kRSize];
+// R_tuv(p, PC), t + u + v <= N (numbered as the Cartesian components of cart.hpp), by the recursion over the auxiliary order from
+// R^(m)_000 = (-2p)^m F_m(p |PC|^2), one order at a time.
+template <int N>
+HFG_INLINE void hermite_r(double p, const double* pc, const double* tab, double* R) {
+    double F[N + 1];
+    boys_eval<N, double>(p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]), tab, 1.0, F);
     double f = 1.0;
-    for (int m = 0; m < N; ++m) f *= -2.0 * p;
-    prev[0] = f * F[N];  // order N: only R_000
-    for (int m = N - 1; m >= 0; --m) {
-        f /= -2.0 * p;
-        cur[0] = f * F[m];
-        const int smax = N - m;
-        for (int s = 1; s <= smax; ++s)
-            for (int t = 0; t <= s; ++t)
-                for (int u = 0; u <= s - t; ++u) {
-                    const int v = s - t - u;
-                    double val;
-                    if (t > 0)
-                        val = (t > 1 ? (t - 1) * prev[ridx(t - 2, u, v)] : 0.0) + pc[0] * prev[ridx(t - 1, u, v)];
-                    else if (u > 0)
-                        val = (u > 1 ? (u - 1) * prev[ridx(t, u - 2, v)] : 0.0) + pc[1] * prev[ridx(t, u - 1, v)];
-                    else
-                        val = (v > 1 ? (v - 1) * prev[ridx(t, u, v - 2)] : 0.0) + pc[2] * prev[ridx(t, u, v - 1)];
-                    cur[ridx(t, u, v)] = val;
-                }
-        for (int k = 0; k < (smax + 1) * (smax + 2) * (smax + 3) / 6; ++k) prev[k] = cur[k];
-    }
-    for (int k = 0; k < (N + 1) * (N + 2) * (N + 3) / 6; ++k) R[k] = prev[k];
+    sfor<N + 1>([&](auto m) {
+        F[m] *= f;
+        f *= -2.0 * p;
+    });
+    double prev[rsize(N)];
+    prev[0] = F[N];
+    sfor<N>([&](auto k) {
+        constexpr int m = N - 1 - k;
+        double cur[rsize(N - m)];
+        cur[0] = F[m];
+        sfor<rsize(N - m) - 1>([&](auto x0) {
+            constexpr int x = x0 + 1, d = gdir(x), x1 = gminus(x, d), n1 = gexp(x1, d);
+            double v = pc[d] * prev[x1];
+            if constexpr (n1 > 0) v += (double)n1 * prev[gminus(x1, d)];
+            cur[x] = v;
+        });
+        sfor<rsize(N - m)>([&](auto x) { prev[x] = cur[x]; });
+    });
+    sfor<rsize(N)>([&](auto x) { R[x] = prev[x]; });
 }
 
-struct PrimPairDev {
+// Hermite coefficients E^{ij}_t of one direction, i <= IM, j <= JM.
+template <int IM, int JM>
+struct Herm {
+    static constexpr int NT = IM + JM + 1;
+    double e[IM + 1][JM + 1][NT];
+    HFG_INLINE void build(double o2p, double pa, double pb) {
+        sfor<IM + 1>([&](auto i) {
+            sfor<JM + 1>([&](auto j) {
+                sfor<i + j + 1>([&](auto t) {
+                    if constexpr (i == 0 && j == 0) {
+                        e[0][0][0] = 1.0;
+                    } else {
+                        constexpr int si = i > 0 ? i - 1 : 0, sj = i > 0 ? (int)j : j - 1;
+                        constexpr int top = si + sj;
+                        double v = 0.0;
+                        if constexpr (t > 0) v += o2p * e[si][sj][t - 1];
+                        if constexpr (t <= top) v += (i > 0 ? pa : pb) * e[si][sj][t];
+                        if constexpr (t + 1 <= top) v += (double)(t + 1) * e[si][sj][t + 1];
+                        e[i][j][t] = v;
+                    }
+                });
+            });
+        });
+    }
+    // coefficient t of (i, j), 0 outside
+    template <int I, int J, int T>
+    HFG_INLINE double at() const {
+        if constexpr (I < 0 || J < 0 || T < 0 || T > I + J)
+            return 0.0;
+        else
+            return e[I][J][T];
+    }
+};
+
+// 1-D overlaps s(i, j), i <= IM, j <= JM, of one direction.
+template <int IM, int JM>
+struct Overlap1 {
+    double s[IM + 1][JM + 1];
+    HFG_INLINE void build(double s00, double o2p, double pa, double pb) {
+        s[0][0] = s00;
+        sfor<IM>([&](auto i) {
+            double v = pa * s[i][0];
+            if constexpr (i > 0) v += (double)(int)i * o2p * s[i - 1][0];
+            s[i + 1][0] = v;
+        });
+        sfor<JM>([&](auto j) {
+            sfor<IM + 1>([&](auto i) {
+                double v = pb * s[i][j];
+                if constexpr (j > 0) v += (double)(int)j * o2p * s[i][j - 1];
+                if constexpr (i > 0) v += (double)(int)i * o2p * s[i - 1][j];
+                s[i][j + 1] = v;
+            });
+        });
+    }
+    // kinetic factor -1/2 <i| d2/dx2 |j> with the ket's exponent b
+    template <int I, int J>
+    HFG_INLINE double kin(double b) const {
+        double v = b * (double)(2 * J + 1) * s[I][J] - 2.0 * b * b * s[I][J + 2];
+        if constexpr (J > 1) v -= 0.5 * (double)(J * (J - 1)) * s[I][J - 2];
+        return v;
+    }
+};
+
+struct PrimPair {
     double a, b, p, P[3], PA[3], PB[3], K;  // K = exp(-ab/p |AB|^2) c_a c_b
 };
 
-__device__ inline PrimPairDev prim_pair_dev(const OneArgs& g, int sa, int i, int sb, int j) {
-    const OneShell A = g.sh[sa], B = g.sh[sb];
+HFG_INLINE PrimPair prim_pair(const OneArgs& g, const OneShell& A, const OneShell& B, int i, int j) {
     const double* ra = g.xyz + 3 * A.atom;
     const double* rb = g.xyz + 3 * B.atom;
-    PrimPairDev pp;
+    PrimPair pp;
     pp.a = g.alpha[A.po + i];
     pp.b = g.alpha[B.po + j];
     pp.p = pp.a + pp.b;
+    const double ip = 1.0 / pp.p;
     double r2 = 0.0;
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        pp.P[d] = (pp.a * ra[d] + pp.b * rb[d]) / pp.p;
+        pp.P[d] = (pp.a * ra[d] + pp.b * rb[d]) * ip;
         pp.PA[d] = pp.P[d] - ra[d];
         pp.PB[d] = pp.P[d] - rb[d];
         r2 += (ra[d] - rb[d]) * (ra[d] - rb[d]);
     }
-    pp.K = exp(-pp.a * pp.b / pp.p * r2) * g.coef[A.po + i] * g.coef[B.po + j];
+    pp.K = exp(-pp.a * pp.b * ip * r2) * g.coef[A.po + i] * g.coef[B.po + j];
     return pp;
 }
 
-template <class E1>
-__device__ inline double s1(const E1& E, double sq, int i, int j) { return (i < 0 || j < 0) ? 0.0 : E.get(i, j, 0) * sq; }
-template <class E1>
-__device__ inline double t1(const E1& E, double sq, double b, int i, int j) {
-    return -0.5 * (j * (j - 1) * s1(E, sq, i, j - 2) - 2.0 * b * (2 * j + 1) * s1(E, sq, i, j) +
-                   4.0 * b * b * s1(E, sq, i, j + 2));
-}
+// Slices of the nuclei per primitive pair, so that a shell pair's items fill its sixteen lanes.
+HFG_INLINE int nuclear_slices(int nprim) { return nprim >= 48 ? 1 : nprim >= 4 ? 4 : kOneLanes; }
 
-// Output-basis block out (na x nb) of a Cartesian block B (nca x ncb): out = Ta^T B Tb (spherical,
-// hfscf's order m = -l..l) or B itself.
-__device__ inline void block_out(int La, int Lb, bool pure, const double* B, double* out) {
-    const int nca = ncart1(La), ncb = ncart1(Lb);
-    if (!pure) {
-        for (int k = 0; k < nca * ncb; ++k) out[k] = B[k];
-        return;
-    }
-    const int nsa = 2 * La + 1, nsb = 2 * Lb + 1;
-    for (int s = 0; s < nsa; ++s) {
-        const SphTerms ta = sph_terms(La, s);
-        for (int t = 0; t < nsb; ++t) {
-            const SphTerms tb = sph_terms(Lb, t);
-            double v = 0.0;
-            for (int x = 0; x < ta.n; ++x)
-                for (int y = 0; y < tb.n; ++y) v += ta.w[x] * tb.w[y] * B[ta.c[x] * ncb + tb.c[y]];
-            out[s * nsb + t] = v;
+template <int LA, int LB>
+__global__ __launch_bounds__(kOneBlock) void oneint_kernel(OneArgs g, const int2* __restrict__ pairs, int npairs) {
+    constexpr int L = LA + LB, ca = ncart(LA), cb = ncart(LB), nab = ca * cb;
+    const int k = blockIdx.x * (kOneBlock / kOneLanes) + threadIdx.x / kOneLanes, ln = threadIdx.x & (kOneLanes - 1);
+    if (k >= npairs) return;  // whole groups of lanes: the shuffles below stay within a group
+    const OneShell A = g.sh[pairs[k].x], B = g.sh[pairs[k].y];
+    double Sb[nab], Tk[nab], Vb[nab];
+    sfor<nab>([&](auto x) { Sb[x] = Tk[x] = Vb[x] = 0.0; });
+    const int nprim = A.np * B.np, nsl = nuclear_slices(nprim);
+    for (int x = ln; x < nprim * nsl; x += kOneLanes) {
+        const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
+        const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
+        if (!(fabs(pp.K) >= kOneTiny)) continue;
+        const double o2p = 0.5 / pp.p;
+        if (sl == 0) {
+            Overlap1<LA, LB + 2> s[3];
+            const double s00 = sqrt(M_PI / pp.p);
+            sfor<3>([&](auto d) { s[d].build(d == 2 ? s00 * pp.K : s00, o2p, pp.PA[d], pp.PB[d]); });
+            sfor<nab>([&](auto ab) {
+                constexpr int ga = ncum(LA - 1) + ab / cb, gb = ncum(LB - 1) + ab % cb;
+                constexpr int ax = gexp(ga, 0), ay = gexp(ga, 1), az = gexp(ga, 2);
+                constexpr int bx = gexp(gb, 0), by = gexp(gb, 1), bz = gexp(gb, 2);
+                const double sx = s[0].s[ax][bx], sy = s[1].s[ay][by], sz = s[2].s[az][bz];
+                Sb[ab] += sx * sy * sz;
+                Tk[ab] += s[0].template kin<ax, bx>(pp.b) * sy * sz + sx * s[1].template kin<ay, by>(pp.b) * sz +
+                          sx * sy * s[2].template kin<az, bz>(pp.b);
+            });
         }
-    }
-}
-
-// Cartesian weight block Wc (nca x ncb) = Ta W_ab Tb^T of the output-basis matrix W (n x n).
-__device__ inline void weight_cart(int La, int Lb, bool pure, const double* W, int n, int oa, int ob, double* Wc) {
-    const int nca = ncart1(La), ncb = ncart1(Lb);
-    if (!pure) {
-        for (int p = 0; p < nca; ++p)
-            for (int q = 0; q < ncb; ++q) Wc[p * ncb + q] = W[(size_t)(oa + p) * n + ob + q];
-        return;
-    }
-    for (int k = 0; k < nca * ncb; ++k) Wc[k] = 0.0;
-    for (int s = 0; s < 2 * La + 1; ++s) {
-        const SphTerms ta = sph_terms(La, s);
-        for (int t = 0; t < 2 * Lb + 1; ++t) {
-            const SphTerms tb = sph_terms(Lb, t);
-            const double w = W[(size_t)(oa + s) * n + ob + t];
-            for (int x = 0; x < ta.n; ++x)
-                for (int y = 0; y < tb.n; ++y) Wc[ta.c[x] * ncb + tb.c[y]] += ta.w[x] * tb.w[y] * w;
-        }
-    }
-}
-
-__device__ inline void scatter(const OneArgs& g, int sa, int sb, const double* blk, double* M) {
-    const OneShell A = g.sh[sa], B = g.sh[sb];
-    const int na = g.pure ? 2 * A.L + 1 : ncart1(A.L), nb = g.pure ? 2 * B.L + 1 : ncart1(B.L);
-    for (int p = 0; p < na; ++p)
-        for (int q = 0; q < nb; ++q) {
-            M[(size_t)(A.ao + p) * g.n + B.ao + q] = blk[p * nb + q];
-            M[(size_t)(B.ao + q) * g.n + A.ao + p] = blk[p * nb + q];
-        }
-}
-
-constexpr int kBlk = 36;  // 6 x 6 Cartesian components of two d shells
-
-// Adds block blk (na x nb) of shell pair (sa, sb) into M with atomics: at (a, b) and, for two
-// different shells, at (b, a) (the block of a shell with itself already covers both).
-__device__ inline void scatter_add(const OneArgs& g, int sa, int sb, const double* blk, double* M) {
-    const OneShell A = g.sh[sa], B = g.sh[sb];
-    const int na = g.pure ? 2 * A.L + 1 : ncart1(A.L), nb = g.pure ? 2 * B.L + 1 : ncart1(B.L);
-    for (int p = 0; p < na; ++p)
-        for (int q = 0; q < nb; ++q) {
-            atomicAdd(&M[(size_t)(A.ao + p) * g.n + B.ao + q], blk[p * nb + q]);
-            if (sa != sb) atomicAdd(&M[(size_t)(B.ao + q) * g.n + A.ao + p], blk[p * nb + q]);
-        }
-}
-
-// S and T of shell pair k (sa >= sb) of the pair list.
-__global__ __launch_bounds__(64) void overlap_kinetic_kernel(OneArgs g) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= g.npairs) return;
-    const int sa = g.pairs[k].x, sb = g.pairs[k].y;
-    const OneShell A = g.sh[sa], B = g.sh[sb];
-    const int nca = ncart1(A.L), ncb = ncart1(B.L);
-    double Sb[kBlk], Tb[kBlk];
-    for (int x = 0; x < kBlk; ++x) Sb[x] = Tb[x] = 0.0;
-    Herm1<kOneMaxL + 1, kOneMaxL + 3> E[3];
-    for (int i = 0; i < A.np; ++i)
-        for (int j = 0; j < B.np; ++j) {
-            const PrimPairDev pp = prim_pair_dev(g, sa, i, sb, j);
-            for (int d = 0; d < 3; ++d) E[d].build(A.L, B.L + 2, pp.p, pp.PA[d], pp.PB[d]);
-            const double sq = sqrt(M_PI / pp.p);
-            for (int x = 0; x < nca; ++x)
-                for (int y = 0; y < ncb; ++y) {
-                    int a[3], b[3];
-                    cart_lmn(A.L, x, a);
-                    cart_lmn(B.L, y, b);
-                    const double sx = s1(E[0], sq, a[0], b[0]), sy = s1(E[1], sq, a[1], b[1]),
-                                 sz = s1(E[2], sq, a[2], b[2]);
-                    const double tx = t1(E[0], sq, pp.b, a[0], b[0]), ty = t1(E[1], sq, pp.b, a[1], b[1]),
-                                 tz = t1(E[2], sq, pp.b, a[2], b[2]);
-                    Sb[x * ncb + y] += pp.K * sx * sy * sz;
-                    Tb[x * ncb + y] += pp.K * (tx * sy * sz + sx * ty * sz + sx * sy * tz);
-                }
-        }
-    double o[kBlk];
-    block_out(A.L, B.L, g.pure, Sb, o);
-    scatter(g, sa, sb, o, g.S);
-    block_out(A.L, B.L, g.pure, Tb, o);
-    scatter(g, sa, sb, o, g.T);
-}
-
-// The attraction of nucleus c in V for shell pair k (one lane per pair and nucleus, added into
-// the zeroed V with atomics).
-__global__ __launch_bounds__(64) void nuclear_kernel(OneArgs g) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)g.npairs * g.natom) return;
-    const int k = (int)(t / g.natom), c = (int)(t - (long long)k * g.natom);
-    const int sa = g.pairs[k].x, sb = g.pairs[k].y;
-    const OneShell A = g.sh[sa], B = g.sh[sb];
-    const int nca = ncart1(A.L), ncb = ncart1(B.L);
-    double Vb[kBlk];
-    for (int x = 0; x < kBlk; ++x) Vb[x] = 0.0;
-    Herm1<kOneMaxL + 1, kOneMaxL + 1> E[3];
-    double R[kRSize];
-    const double zc = g.Z[c];
-    for (int i = 0; i < A.np; ++i)
-        for (int j = 0; j < B.np; ++j) {
-            const PrimPairDev pp = prim_pair_dev(g, sa, i, sb, j);
-            for (int d = 0; d < 3; ++d) E[d].build(A.L, B.L, pp.p, pp.PA[d], pp.PB[d]);
-            const double pre = 2.0 * M_PI / pp.p * pp.K;
+        double h[rsize(L)];  // sum_C -Z_C R_tuv
+        sfor<rsize(L)>([&](auto t) { h[t] = 0.0; });
+        for (int c = sl; c < g.natom; c += nsl) {
             const double pc[3] = {pp.P[0] - g.xyz[3 * c], pp.P[1] - g.xyz[3 * c + 1], pp.P[2] - g.xyz[3 * c + 2]};
-            hermite_r(A.L + B.L, pp.p, pc, g.boys, R);
-            for (int x = 0; x < nca; ++x)
-                for (int y = 0; y < ncb; ++y) {
-                    int a[3], b[3];
-                    cart_lmn(A.L, x, a);
-                    cart_lmn(B.L, y, b);
-                    double acc = 0.0;
-                    for (int tt = 0; tt <= a[0] + b[0]; ++tt)
-                        for (int u = 0; u <= a[1] + b[1]; ++u)
-                            for (int v = 0; v <= a[2] + b[2]; ++v)
-                                acc += E[0].get(a[0], b[0], tt) * E[1].get(a[1], b[1], u) * E[2].get(a[2], b[2], v) *
-                                       R[ridx(tt, u, v)];
-                    Vb[x * ncb + y] -= zc * pre * acc;
-                }
+            const double z = g.Z[c];
+            double R[rsize(L)];
+            hermite_r<L>(pp.p, pc, g.boys, R);
+            sfor<rsize(L)>([&](auto t) { h[t] -= z * R[t]; });
         }
-    double o[kBlk];
-    block_out(A.L, B.L, g.pure, Vb, o);
-    scatter_add(g, sa, sb, o, g.V);
+        const double pre = 4.0 * M_PI * o2p * pp.K;  // 2 pi / p
+        Herm<LA, LB> E[3];
+        sfor<3>([&](auto d) { E[d].build(o2p, pp.PA[d], pp.PB[d]); });
+        sfor<nab>([&](auto ab) {
+            constexpr int ga = ncum(LA - 1) + ab / cb, gb = ncum(LB - 1) + ab % cb;
+            constexpr int nx = gexp(ga, 0) + gexp(gb, 0) + 1, ny = gexp(ga, 1) + gexp(gb, 1) + 1,
+                          nz = gexp(ga, 2) + gexp(gb, 2) + 1;
+            double v = 0.0;
+            sfor<nx>([&](auto t) {
+                sfor<ny>([&](auto u) {
+                    double w = 0.0;
+                    sfor<nz>([&](auto q) { w += E[2].e[gexp(ga, 2)][gexp(gb, 2)][q] * h[ridx(t, u, q)]; });
+                    v += E[0].e[gexp(ga, 0)][gexp(gb, 0)][t] * E[1].e[gexp(ga, 1)][gexp(gb, 1)][u] * w;
+                });
+            });
+            Vb[ab] += pre * v;
+        });
+    }
+    // the group's sums, each element written by one lane to both triangles
+    const int oa = g.cart_off[pairs[k].x], ob = g.cart_off[pairs[k].y];
+    sfor<nab>([&](auto ab) {
+        double s = Sb[ab], t = Tk[ab], v = Vb[ab];
+#pragma unroll
+        for (int o = kOneLanes / 2; o > 0; o >>= 1) {
+            s += __shfl_xor(s, o);
+            t += __shfl_xor(t, o);
+            v += __shfl_xor(v, o);
+        }
+        if ((ab & (kOneLanes - 1)) == ln) {
+            const size_t e = (size_t)(oa + ab / cb) * g.ncart + ob + ab % cb;
+            const size_t f = (size_t)(ob + ab % cb) * g.ncart + oa + ab / cb;
+            g.S[e] = s;
+            g.S[f] = s;
+            g.T[e] = t;
+            g.T[f] = t;
+            g.V[e] = v;
+            g.V[f] = v;
+        }
+    });
 }
 
-// One-electron gradient terms of shell pair (sa, sb) and its mirror (sb, sa) (the sum over i, j of
-// the gradient formula runs over both orders), added into grad with atomics:
-//   2 D_ab d(T + V)_ab/dX - 2 Q_ab dS_ab/dX.
-__global__ __launch_bounds__(64) void oneint_grad_kernel(OneArgs g, const double* D, const double* Q, double* grad) {
-    // one lane per shell pair (sa >= sb) and part: part natom = overlap and kinetic terms, part
-    // c < natom = the attraction of nucleus c. D and Q are symmetric, so the ordered pair (sb, sa)
-    // adds what (sa, sb) adds: a pair of two shells counts twice.
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int parts = g.natom + 1;
-    if (tid >= (long long)g.npairs * parts) return;
-    const int k = (int)(tid / parts), part = (int)(tid - (long long)k * parts);
-    const int sa = g.pairs[k].x, sb = g.pairs[k].y;
-    const OneShell A = g.sh[sa], B = g.sh[sb];
-    const int nca = ncart1(A.L), ncb = ncart1(B.L);
-    double WD[kBlk], WQ[kBlk];
-    weight_cart(A.L, B.L, g.pure, D, g.n, A.ao, B.ao, WD);
-    weight_cart(A.L, B.L, g.pure, Q, g.n, A.ao, B.ao, WQ);
-    if (sa != sb)
-        for (int x = 0; x < nca * ncb; ++x) {
-            WD[x] *= 2.0;
-            WQ[x] *= 2.0;
-        }
-    double gA[3] = {0.0, 0.0, 0.0}, gB[3] = {0.0, 0.0, 0.0};
-    Herm1<kOneMaxL + 2, kOneMaxL + 4> E[3];
-    double R[kRSize];
-    for (int i = 0; i < A.np; ++i)
-        for (int j = 0; j < B.np; ++j) {
-            const PrimPairDev pp = prim_pair_dev(g, sa, i, sb, j);
-            for (int d = 0; d < 3; ++d) E[d].build(A.L + 1, B.L + 3, pp.p, pp.PA[d], pp.PB[d]);
-            const double sq = sqrt(M_PI / pp.p);
-            // overlap and kinetic: d/dA = 2a |a+1> - a_x |a-1>; d/dB = -d/dA
-            if (part == g.natom)
-            for (int x = 0; x < nca; ++x)
-                for (int y = 0; y < ncb; ++y) {
-                    const double wd = WD[x * ncb + y], wq = WQ[x * ncb + y];
-                    if (wd == 0.0 && wq == 0.0) continue;
-                    int a[3], b[3];
-                    cart_lmn(A.L, x, a);
-                    cart_lmn(B.L, y, b);
-                    double s[3], t[3], ds[3], dt[3];
-                    for (int d = 0; d < 3; ++d) {
-                        s[d] = s1(E[d], sq, a[d], b[d]);
-                        t[d] = t1(E[d], sq, pp.b, a[d], b[d]);
-                        ds[d] = 2.0 * pp.a * s1(E[d], sq, a[d] + 1, b[d]) - (a[d] > 0 ? a[d] * s1(E[d], sq, a[d] - 1, b[d]) : 0.0);
-                        dt[d] = 2.0 * pp.a * t1(E[d], sq, pp.b, a[d] + 1, b[d]) -
-                                (a[d] > 0 ? a[d] * t1(E[d], sq, pp.b, a[d] - 1, b[d]) : 0.0);
-                    }
-                    for (int d = 0; d < 3; ++d) {
-                        const int e1 = (d + 1) % 3, e2 = (d + 2) % 3;
-                        const double dS = pp.K * ds[d] * s[e1] * s[e2];
-                        const double dT = pp.K * (dt[d] * s[e1] * s[e2] + ds[d] * t[e1] * s[e2] + ds[d] * s[e1] * t[e2]);
-                        const double v = -2.0 * wq * dS + 2.0 * wd * dT;
+// Gradient terms 2 D_ab d(T + V)_ab/dX - 2 Q_ab dS_ab/dX of the shell pairs, D and Q Cartesian and
+// symmetric: a pair of two shells counts twice for its mirror. The workgroup's sums per nucleus
+// live in LDS (in grad itself beyond kOneLdsAtoms nuclei); the lanes start at different nuclei, so
+// their LDS additions fall on different addresses.
+template <int LA, int LB>
+__global__ __launch_bounds__(kOneBlock) void oneint_grad_kernel(OneArgs g, const int2* __restrict__ pairs, int npairs,
+                                                                const double* __restrict__ D, const double* __restrict__ Q,
+                                                                double* grad) {
+    constexpr int L = LA + LB, ca = ncart(LA), cb = ncart(LB), nab = ca * cb;
+    extern __shared__ double gs[];
+    const bool lds = g.natom <= kOneLdsAtoms;
+    auto add = [&](int e, double v) {
+        if (lds)
+            atomicAdd(&gs[e], v);
+        else
+            unsafeAtomicAdd(&grad[e], v);
+    };
+    if (lds)
+        for (int x = threadIdx.x; x < 3 * g.natom; x += kOneBlock) gs[x] = 0.0;
+    __syncthreads();
+    const int ln = threadIdx.x & (kOneLanes - 1), per = kOneBlock / kOneLanes;
+    for (int k = blockIdx.x * per + threadIdx.x / kOneLanes; k < npairs; k += gridDim.x * per) {
+        const int sa = pairs[k].x, sb = pairs[k].y;
+        const OneShell A = g.sh[sa], B = g.sh[sb];
+        // weights of the block (larger shell index, smaller) as it is stored; read again at each use,
+        // which leaves the registers to the d pairs' tables
+        const double f0 = sa == sb ? 2.0 : 4.0;
+        const bool in_order = sa >= sb;
+        const size_t w0 = in_order ? (size_t)g.cart_off[sa] * g.ncart + g.cart_off[sb]
+                                   : (size_t)g.cart_off[sb] * g.ncart + g.cart_off[sa];
+        const int wr = in_order ? g.ncart : 1, wc = in_order ? 1 : g.ncart;
+        auto weight = [&](const double* M, int ab) { return f0 * M[w0 + (size_t)(ab / cb) * wr + (ab % cb) * wc]; };
+        double gA[3] = {0.0, 0.0, 0.0}, gB[3] = {0.0, 0.0, 0.0};
+        const int nprim = A.np * B.np, nsl = nuclear_slices(nprim);
+        for (int x = ln; x < nprim * nsl; x += kOneLanes) {
+            const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
+            const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
+            if (!(fabs(pp.K) >= kOneTiny)) continue;
+            const double o2p = 0.5 / pp.p, ta = 2.0 * pp.a;
+            if (sl == 0) {
+                Overlap1<LA + 1, LB + 2> s[3];
+                const double s00 = sqrt(M_PI / pp.p);
+                sfor<3>([&](auto d) { s[d].build(d == 2 ? s00 * pp.K : s00, o2p, pp.PA[d], pp.PB[d]); });
+                sfor<nab>([&](auto ab) {
+                    constexpr int ga = ncum(LA - 1) + ab / cb, gb = ncum(LB - 1) + ab % cb;
+                    double sv[3], tv[3], ds[3], dt[3];
+                    const double wd = weight(D, ab), wq = weight(Q, ab);
+                    sfor<3>([&](auto d) {
+                        constexpr int ia = gexp(ga, d), jb = gexp(gb, d);
+                        sv[d] = s[d].s[ia][jb];
+                        tv[d] = s[d].template kin<ia, jb>(pp.b);
+                        ds[d] = ta * s[d].s[ia + 1][jb];
+                        dt[d] = ta * s[d].template kin<ia + 1, jb>(pp.b);
+                        if constexpr (ia > 0) {
+                            ds[d] -= (double)ia * s[d].s[ia - 1][jb];
+                            dt[d] -= (double)ia * s[d].template kin<ia - 1, jb>(pp.b);
+                        }
+                    });
+                    sfor<3>([&](auto d) {
+                        constexpr int e1 = (d + 1) % 3, e2 = (d + 2) % 3;
+                        const double dS = ds[d] * sv[e1] * sv[e2];
+                        const double dT = dt[d] * sv[e1] * sv[e2] + ds[d] * (tv[e1] * sv[e2] + sv[e1] * tv[e2]);
+                        const double v = wd * dT - wq * dS;
                         gA[d] += v;
                         gB[d] -= v;
-                    }
-                }
-            // nuclear attraction: bra and ket shifts, and the operator's centre by translational
-            // invariance (dC = -(dA + dB))
-            const double pre = 2.0 * M_PI / pp.p * pp.K;
-            if (part < g.natom) {
-                const int c = part;
-                const double pc[3] = {pp.P[0] - g.xyz[3 * c], pp.P[1] - g.xyz[3 * c + 1], pp.P[2] - g.xyz[3 * c + 2]};
-                hermite_r(A.L + B.L + 1, pp.p, pc, g.boys, R);
-                auto vint = [&](const int* a, const int* b) {
-                    if (a[0] < 0 || a[1] < 0 || a[2] < 0 || b[0] < 0 || b[1] < 0 || b[2] < 0) return 0.0;
-                    double acc = 0.0;
-                    for (int t = 0; t <= a[0] + b[0]; ++t)
-                        for (int u = 0; u <= a[1] + b[1]; ++u)
-                            for (int v = 0; v <= a[2] + b[2]; ++v)
-                                acc += E[0].get(a[0], b[0], t) * E[1].get(a[1], b[1], u) * E[2].get(a[2], b[2], v) *
-                                       R[ridx(t, u, v)];
-                    return -g.Z[c] * pre * acc;
-                };
-                double gc[3] = {0.0, 0.0, 0.0};
-                for (int x = 0; x < nca; ++x)
-                    for (int y = 0; y < ncb; ++y) {
-                        const double wd = WD[x * ncb + y];
-                        if (wd == 0.0) continue;
-                        int a0[3], b0[3];
-                        cart_lmn(A.L, x, a0);
-                        cart_lmn(B.L, y, b0);
-                        for (int d = 0; d < 3; ++d) {
-                            int ap[3] = {a0[0], a0[1], a0[2]}, am[3] = {a0[0], a0[1], a0[2]};
-                            int bp[3] = {b0[0], b0[1], b0[2]}, bm[3] = {b0[0], b0[1], b0[2]};
-                            ap[d] += 1;
-                            am[d] -= 1;
-                            bp[d] += 1;
-                            bm[d] -= 1;
-                            const double dA = 2.0 * pp.a * vint(ap, b0) - (a0[d] ? a0[d] * vint(am, b0) : 0.0);
-                            const double dB = 2.0 * pp.b * vint(a0, bp) - (b0[d] ? b0[d] * vint(a0, bm) : 0.0);
-                            gA[d] += 2.0 * wd * dA;
-                            gB[d] += 2.0 * wd * dB;
-                            gc[d] -= 2.0 * wd * (dA + dB);
-                        }
-                    }
-                for (int d = 0; d < 3; ++d)
-                    if (gc[d] != 0.0) atomicAdd(&grad[3 * c + d], gc[d]);
+                    });
+                });
             }
+            // Hermite density of the primitive pair
+            const double pre = 4.0 * M_PI * o2p * pp.K;
+            Herm<LA + 1, LB> E[3];
+            sfor<3>([&](auto d) { E[d].build(o2p, pp.PA[d], pp.PB[d]); });
+            double w[rsize(L)];
+            sfor<rsize(L)>([&](auto t) { w[t] = 0.0; });
+            sfor<nab>([&](auto ab) {
+                constexpr int ga = ncum(LA - 1) + ab / cb, gb = ncum(LB - 1) + ab % cb;
+                const double f = pre * weight(D, ab);
+                sfor<gexp(ga, 0) + gexp(gb, 0) + 1>([&](auto t) {
+                    const double ft = f * E[0].e[gexp(ga, 0)][gexp(gb, 0)][t];
+                    sfor<gexp(ga, 1) + gexp(gb, 1) + 1>([&](auto u) {
+                        const double fu = ft * E[1].e[gexp(ga, 1)][gexp(gb, 1)][u];
+                        sfor<gexp(ga, 2) + gexp(gb, 2) + 1>(
+                            [&](auto q) { w[ridx(t, u, q)] += fu * E[2].e[gexp(ga, 2)][gexp(gb, 2)][q]; });
+                    });
+                });
+            });
+            double h[rsize(L + 1)];  // sum_C -Z_C R_tuv
+            sfor<rsize(L + 1)>([&](auto t) { h[t] = 0.0; });
+            const int cnt = (g.natom - sl + nsl - 1) / nsl;
+            int c = cnt > 0 ? sl + nsl * ((int)threadIdx.x % cnt) : 0;
+            for (int n = 0; n < cnt; ++n) {
+                const double pc[3] = {pp.P[0] - g.xyz[3 * c], pp.P[1] - g.xyz[3 * c + 1], pp.P[2] - g.xyz[3 * c + 2]};
+                const double z = g.Z[c];
+                double R[rsize(L + 1)];
+                hermite_r<L + 1>(pp.p, pc, g.boys, R);
+                double dc[3] = {0.0, 0.0, 0.0};
+                sfor<rsize(L)>([&](auto t) { sfor<3>([&](auto d) { dc[d] += w[t] * R[gplus(t, d)]; }); });
+                sfor<rsize(L + 1)>([&](auto t) { h[t] -= z * R[t]; });
+#pragma unroll
+                for (int d = 0; d < 3; ++d) add(3 * c + d, z * dc[d]);
+                c += nsl;
+                if (c >= g.natom) c = sl;
+            }
+            // d/dP, and d/dA by the shifts of the bra; d/dB = d/dP - d/dA
+            sfor<3>([&](auto d) {
+                double dp = 0.0, da = 0.0;
+                sfor<rsize(L)>([&](auto t) { dp += w[t] * h[gplus(t, d)]; });
+                sfor<nab>([&](auto ab) {
+                    constexpr int ga = ncum(LA - 1) + ab / cb, gb = ncum(LB - 1) + ab % cb;
+                    constexpr int e1 = (d + 1) % 3, e2 = (d + 2) % 3;
+                    constexpr int ia = gexp(ga, d), jb = gexp(gb, d);
+                    double v = 0.0;
+                    sfor<ia + jb + 2>([&](auto t) {
+                        double ed = ta * E[d].template at<ia + 1, jb, t>();
+                        if constexpr (ia > 0) ed -= (double)ia * E[d].template at<ia - 1, jb, t>();
+                        double q1 = 0.0;
+                        sfor<gexp(ga, e1) + gexp(gb, e1) + 1>([&](auto u) {
+                            double q2 = 0.0;
+                            sfor<gexp(ga, e2) + gexp(gb, e2) + 1>([&](auto q) {
+                                constexpr int tu[3] = {d == 0 ? (int)t : e1 == 0 ? (int)u : (int)q,
+                                                       d == 1 ? (int)t : e1 == 1 ? (int)u : (int)q,
+                                                       d == 2 ? (int)t : e1 == 2 ? (int)u : (int)q};
+                                q2 += E[e2].e[gexp(ga, e2)][gexp(gb, e2)][q] * h[ridx(tu[0], tu[1], tu[2])];
+                            });
+                            q1 += E[e1].e[gexp(ga, e1)][gexp(gb, e1)][u] * q2;
+                        });
+                        v += ed * q1;
+                    });
+                    da += weight(D, ab) * v;
+                });
+                da *= pre;
+                gA[d] += da;
+                gB[d] += dp - da;
+            });
         }
-    for (int d = 0; d < 3; ++d) {
-        atomicAdd(&grad[3 * A.atom + d], gA[d]);
-        atomicAdd(&grad[3 * B.atom + d], gB[d]);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+#pragma unroll
+            for (int o = kOneLanes / 2; o > 0; o >>= 1) {
+                gA[d] += __shfl_xor(gA[d], o);
+                gB[d] += __shfl_xor(gB[d], o);
+            }
+        if (ln < 3) {
+            const double va = ln == 0 ? gA[0] : ln == 1 ? gA[1] : gA[2], vb = ln == 0 ? gB[0] : ln == 1 ? gB[1] : gB[2];
+            add(3 * A.atom + ln, va);
+            add(3 * B.atom + ln, vb);
+        }
+    }
+    __syncthreads();
+    if (lds)
+        for (int x = threadIdx.x; x < 3 * g.natom; x += kOneBlock) unsafeAtomicAdd(&grad[x], gs[x]);
+}
+
+// Output-basis matrices from the Cartesian ones (blockIdx.y: S, T, V): one thread per element.
+__global__ __launch_bounds__(256) void from_cart_kernel(const double* __restrict__ Mc, int nc, const SphTerms* __restrict__ terms,
+                                                        int n, double* __restrict__ M) {
+    const double* src = Mc + (size_t)blockIdx.y * nc * nc;
+    double* dst = M + (size_t)blockIdx.y * n * n;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n * n; e += gridDim.x * 256) {
+        const int i = e / n, j = e - i * n;
+        const SphTerms ti = terms[i], tj = terms[j];
+        double v = 0.0;
+        for (int x = 0; x < ti.n; ++x)
+            for (int y = 0; y < tj.n; ++y) v += ti.w[x] * tj.w[y] * src[(size_t)ti.c[x] * nc + tj.c[y]];
+        dst[e] = v;
     }
 }
+
+constexpr int kClassLa[6] = {2, 2, 2, 1, 1, 0}, kClassLb[6] = {2, 1, 0, 1, 0, 0};
+
+// Shell pairs by class, L(x) >= L(y); first[k]..first[k + 1] are those of class k.
+std::vector<int2> pairs_by_class(const hfg_ctx* c, int* first) {
+    std::vector<int> of_l[3];
+    for (int s = 0; s < c->nshell; ++s) of_l[c->L[s]].push_back(s);
+    std::vector<int2> out;
+    out.reserve((size_t)c->nshell * (c->nshell + 1) / 2);
+    for (int k = 0; k < 6; ++k) {
+        first[k] = (int)out.size();
+        const bool same = kClassLa[k] == kClassLb[k];
+        for (int a : of_l[kClassLa[k]])
+            for (int b : of_l[kClassLb[k]]) {
+                if (same && b > a) break;
+                out.push_back(make_int2(a, b));
+            }
+    }
+    first[6] = (int)out.size();
+    return out;
+}
+
+// The classes as (la, lb, index, stream): (ss|, the longest, on the main stream, the others on two
+// side streams of about its length.
+#define HFG_ONE_CLASSES(X) X(1, 0, 4, 1) X(1, 1, 3, 2) X(0, 0, 5, 0) X(2, 2, 0, 1) X(2, 0, 2, 2) X(2, 1, 1, 2)
+
+// The main stream and the two side streams that the classes run on, forked here.
+struct OneStreams {
+    hipStream_t s[3];
+    hfg_ctx* c;
+    hipError_t fork(hfg_ctx* ctx) {
+        c = ctx;
+        s[0] = c->stream;
+        s[1] = c->side[0];
+        s[2] = c->nside > 1 ? c->side[1] : c->side[0];
+        hipError_t e = hipEventRecord(c->ev_fork, s[0]);
+        for (int k = 1; k < 3 && e == hipSuccess; ++k) e = hipStreamWaitEvent(s[k], c->ev_fork, 0);
+        return e;
+    }
+    hipError_t join() {
+        hipError_t e = hipGetLastError();
+        for (int k = 0; k < std::min(2, c->nside) && e == hipSuccess; ++k) {
+            e = hipEventRecord(c->ev_join[k], c->side[k]);
+            if (e == hipSuccess) e = hipStreamWaitEvent(s[0], c->ev_join[k], 0);
+        }
+        return e;
+    }
+};
 
 }  // namespace
 
-hipError_t launch_oneint(const OneArgs& g, hipStream_t s) {
-    if (g.npairs == 0) return hipSuccess;
-    hipError_t e = hipMemsetAsync(g.V, 0, (size_t)g.n * g.n * sizeof(double), s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(overlap_kinetic_kernel, dim3((g.npairs + 63) / 64), dim3(64), 0, s, g);
-    const long long nv = (long long)g.npairs * g.natom;
-    hipLaunchKernelGGL(nuclear_kernel, dim3((unsigned)((nv + 63) / 64)), dim3(64), 0, s, g);
-    return hipGetLastError();
+// S, T, V over the Cartesian functions (g.S, g.T, g.V).
+static hipError_t launch_oneint(hfg_ctx* c, const OneArgs& g, const int2* pairs, const int* first) {
+    constexpr int per = kOneBlock / kOneLanes;
+    OneStreams st;
+    if (hipError_t e = st.fork(c)) return e;
+#define HFG_RUN(A, B, K, S)                                                                                       \
+    if (const int n = first[K + 1] - first[K])                                                                    \
+        hipLaunchKernelGGL((oneint_kernel<A, B>), dim3((n + per - 1) / per), dim3(kOneBlock), 0, st.s[S], g,       \
+                           pairs + first[K], n);
+    HFG_ONE_CLASSES(HFG_RUN)
+#undef HFG_RUN
+    return st.join();
 }
 
-hipError_t launch_oneint_grad(const OneArgs& g, const double* D, const double* Q, double* grad, hipStream_t s) {
-    const long long n = (long long)g.npairs * (g.natom + 1);
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(oneint_grad_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, g, D, Q, grad);
-    return hipGetLastError();
+static hipError_t launch_oneint_grad(hfg_ctx* c, const OneArgs& g, const int2* pairs, const int* first, const double* D,
+                                     const double* Q, double* grad) {
+    constexpr int per = kOneBlock / kOneLanes;
+    OneStreams st;
+    if (hipError_t e = st.fork(c)) return e;
+    const size_t lds = g.natom <= kOneLdsAtoms ? 3 * sizeof(double) * g.natom : 0;
+    // at most 1024 workgroups per class, so that their flushes stay few
+#define HFG_RUN(A, B, K, S)                                                                                         \
+    if (const int n = first[K + 1] - first[K])                                                                      \
+        hipLaunchKernelGGL((oneint_grad_kernel<A, B>), dim3(std::min((n + per - 1) / per, 1024)), dim3(kOneBlock), lds, \
+                           st.s[S], g, pairs + first[K], n, D, Q, grad);
+    HFG_ONE_CLASSES(HFG_RUN)
+#undef HFG_RUN
+    return st.join();
 }
 
 }  // namespace hfg
@@ -462,9 +528,8 @@ int one_upload(hfg_ctx* c, hfg::OneArgs& g) {
     g.Z = c->d_one_Z.p;
     g.boys = c->d_boys.p;
     g.natom = c->natom;
-    g.nshell = c->nshell;
-    g.n = c->nbf;
-    g.pure = c->pure ? 1 : 0;
+    g.ncart = c->ncart;
+    g.cart_off = c->d_cart_off.p;
     return HFG_OK;
 }
 
@@ -476,21 +541,34 @@ int hfg_oneint(hfg_ctx* c, double* S, double* T, double* V) {
     if (!c) return HFG_ERR_ARG;
     hfg::OneArgs g;
     if (int r = hfg::one_upload(c, g)) return r;
-    std::vector<int2> pairs;
-    for (int a = 0; a < c->nshell; ++a)
-        for (int b = 0; b <= a; ++b) pairs.push_back(make_int2(a, b));
+    int first[7];
+    const std::vector<int2> pairs = hfg::pairs_by_class(c, first);
     HFG_CHECK(c, c->d_one_pairs.upload(pairs, c->stream));
-    const size_t nn = (size_t)c->nbf * c->nbf;
-    HFG_CHECK(c, c->d_one_buf.ensure(3 * nn));
-    g.pairs = c->d_one_pairs.p;
-    g.npairs = (int)pairs.size();
+    const size_t nn = (size_t)c->nbf * c->nbf, cc = (size_t)c->ncart * c->ncart;
+    HFG_CHECK(c, c->d_one_buf.ensure(3 * cc + (c->pure ? 3 * nn : 0)));
     g.S = c->d_one_buf.p;
-    g.T = g.S + nn;
-    g.V = g.T + nn;
-    HFG_CHECK(c, hfg::launch_oneint(g, c->stream));
+    g.T = g.S + cc;
+    g.V = g.T + cc;
+    HFG_CHECK(c, hfg::launch_oneint(c, g, c->d_one_pairs.p, first));
+    const double* res = g.S;  // a Cartesian basis has them already
+    std::vector<hfg::SphTerms> terms(c->pure ? c->nbf : 0);
+    if (c->pure) {
+        for (int s = 0; s < c->nshell; ++s)
+            for (int k = 0; k < hfg::nfun(c->L[s], true); ++k) {
+                hfg::SphTerms t = hfg::sph_terms(c->L[s], k);
+                for (int x = 0; x < t.n; ++x) t.c[x] += c->cart_off[s];
+                terms[c->pure_off[s] + k] = t;
+            }
+        HFG_CHECK(c, c->d_one_terms.upload(terms, c->stream));
+        double* dst = g.S + 3 * cc;
+        hipLaunchKernelGGL(hfg::from_cart_kernel, dim3((unsigned)std::min<size_t>(1024, (nn + 255) / 256), 3), dim3(256), 0,
+                           c->stream, g.S, c->ncart, c->d_one_terms.p, c->nbf, dst);
+        HFG_CHECK(c, hipGetLastError());
+        res = dst;
+    }
     double* out[3] = {S, T, V};
     for (int k = 0; k < 3; ++k)
-        if (out[k]) HFG_CHECK(c, hipMemcpyAsync(out[k], g.S + k * nn, nn * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        if (out[k]) HFG_CHECK(c, hipMemcpyAsync(out[k], res + k * nn, nn * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     return HFG_OK;
 }
@@ -500,22 +578,27 @@ int hfg_oneint_gradient(hfg_ctx* c, const double* D, const double* Q, double* gr
     if (!D || !Q || !grad) return one_fail(c, HFG_ERR_ARG, "hfg_oneint_gradient: null argument");
     hfg::OneArgs g;
     if (int r = hfg::one_upload(c, g)) return r;
-    std::vector<int2> pairs;
-    for (int a = 0; a < c->nshell; ++a)
-        for (int b = 0; b <= a; ++b) pairs.push_back(make_int2(a, b));
+    int first[7];
+    const std::vector<int2> pairs = hfg::pairs_by_class(c, first);
     HFG_CHECK(c, c->d_one_pairs.upload(pairs, c->stream));
-    g.pairs = c->d_one_pairs.p;
-    g.npairs = (int)pairs.size();
-    const size_t nn = (size_t)c->nbf * c->nbf;
+    const size_t nn = (size_t)c->nbf * c->nbf, cc = (size_t)c->ncart * c->ncart;
     const int nout = 3 * c->natom;
-    HFG_CHECK(c, c->d_one_buf.ensure(2 * nn + nout));
+    HFG_CHECK(c, c->d_one_buf.ensure(2 * nn + nout + (c->pure ? 2 * cc : 0)));
     double* dD = c->d_one_buf.p;
     double* dQ = dD + nn;
     double* dg = dQ + nn;
     HFG_CHECK(c, hipMemcpyAsync(dD, D, nn * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HFG_CHECK(c, hipMemcpyAsync(dQ, Q, nn * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HFG_CHECK(c, hipMemcpyAsync(dg, grad, nout * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HFG_CHECK(c, hfg::launch_oneint_grad(g, dD, dQ, dg, c->stream));
+    if (c->pure) {
+        double* cart = dg + nout;
+        for (int k = 0; k < 2; ++k)
+            HFG_CHECK(c, hfg::launch_to_cart(k ? dQ : dD, c->d_mols.p, c->d_mol_cart.p, 1, c->max_ncart, c->d_cart_terms.p,
+                                             cart + k * cc, c->stream));
+        dD = cart;
+        dQ = cart + cc;
+    }
+    HFG_CHECK(c, hfg::launch_oneint_grad(c, g, c->d_one_pairs.p, first, dD, dQ, dg));
     HFG_CHECK(c, hipMemcpyAsync(grad, dg, nout * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     return HFG_OK;
