@@ -20,7 +20,8 @@
 #include "misc.hpp"
 #include "noalloc.hpp"
 #include "private_segments.hpp"
-#include "rys.hpp"
+#include "rys_grad.hpp"
+#include "rys_jk.hpp"
 
 using namespace hfg;
 
@@ -46,25 +47,26 @@ hipStream_t shared_scratch_stream(int device) {
     return streams[device];
 }
 
-// Streams and launch order of the class launches (J/K, or the gradient of a precision when grad): the classes
+// Streams and launch order of a precision's class launches (J/K, or the gradient when grad): the classes
 // of the shared stream (on_shared_stream) run there (-1); the others are balanced over the side
 // streams, onto the least loaded one, by the weights w (the FLOP model at set-up, the measured
 // kernel times after autotuning). The launch order is the cooperative-kernel classes first (one
 // quartet per workgroup at a time: few workgroups on long serial chains, whose latency then
 // hides under the wide launches instead of trailing the build), then heaviest first.
 void assign_streams(hfg_ctx* c, bool grad, bool mixed, const std::vector<double>& w) {
-    std::vector<int>& map = grad ? c->grad_stream[mixed ? 1 : 0] : c->class_stream;
+    std::vector<int>& map = (grad ? c->grad_stream : c->class_stream)[mixed ? 1 : 0];
     map.assign(c->classes.size(), 0);
     std::vector<size_t> ord(c->classes.size());
     std::iota(ord.begin(), ord.end(), 0);
     auto coop = [&](size_t k) {
-        return grad ? c->classes[k].gcoop && !grad_on_rys(c, c->classes[k], mixed) : c->classes[k].coop;
+        const ClassWork& cw = c->classes[k];
+        return grad ? cw.gcoop && !grad_on_rys(c, cw, mixed) : cw.coop && !jk_on_rys(c, cw, mixed);
     };
     std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) {
         if (coop(x) != coop(y)) return coop(x);
         return w[x] > w[y];
     });
-    std::vector<int>& order = grad ? c->grad_order[mixed ? 1 : 0] : c->class_order;
+    std::vector<int>& order = (grad ? c->grad_order : c->class_order)[mixed ? 1 : 0];
     order.assign(ord.begin(), ord.end());
     // the balance is over hardware queues: side streams on one queue count as one, the first of
     // them takes the queue's classes, and a queue shared with the shared stream starts with the
@@ -908,8 +910,10 @@ int setup_geometry(hfg_ctx* c) {
             wj.push_back(cw.jk_flops());
             wg.push_back(cw.grad_flops);
         }
-        assign_streams(c, false, false, wj);
-        for (bool mixed : {false, true}) assign_streams(c, true, mixed, wg);
+        for (bool mixed : {false, true}) {
+            assign_streams(c, false, mixed, wj);
+            assign_streams(c, true, mixed, wg);
+        }
     }
     // gather lists (one output tile per block pair) and per-molecule item lists
     std::vector<std::vector<GatherEntry>> lj(nbp), lk(nbp);
@@ -1039,6 +1043,7 @@ int setup_geometry(hfg_ctx* c) {
         }
         HFG_CHECK(c, c->d_mol_cart.upload(mc, c->stream));
         HFG_CHECK(c, c->d_cart_terms.upload(terms, c->stream));
+        if (c->pure) HFG_CHECK(c, c->d_Dc.ensure(c->nc_total));  // here, so that a build allocates nothing
         HFG_CHECK(c, c->d_shell_ao.upload(ao, c->stream));
         HFG_CHECK(c, c->d_shell_nf.upload(nf, c->stream));
         HFG_CHECK(c, c->d_shell_mol.upload(c->shell_mol, c->stream));
@@ -1134,6 +1139,8 @@ int enqueue_classes(hfg_ctx* c, hipStream_t main, bool dscreen, bool timed, Clas
     a.slab = buf.slab;
     a.dmax = c->d_dmax.p;
     a.dtol = dscreen ? c->opt.density_tol : 0.0;
+    if (set != ClassSet::Shared)
+        if (int r = hfg::make_cart_density(c, buf.D, main)) return r;
     const int ncls = (int)c->classes.size(), nshared = shared_class_count(c, false);
     if (set != ClassSet::Shared) HFG_CHECK(c, launch_zero_ints(buf.queue + nshared, ncls - nshared, main));
     bool shared_zeroed = false;
@@ -1333,6 +1340,10 @@ void layout_molecules(hfg_ctx* c) {
 hipError_t hfg::launch_jk_class(hfg_ctx* c, const ClassWork& cw, const JkArgs& a, LaunchShape sh, hipStream_t st) {
     const int mixed = c->opt.precision == HFG_MIXED ? 1 : 0;
     if (cw.gc) return launch_jk_gc(cw.la, cw.lb, cw.lc, cw.ld, c->pure, mixed, a, c->gc_args, (int)cw.gc_items.size(), sh, st);
+    if (jk_on_rys(c, cw, mixed != 0)) {
+        const RysJkArgs r{a, c->rys, c->pure ? c->d_Dc.p : a.D, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
+        return launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, r, (int)cw.items.size(), sh, st);
+    }
     if (cw.coop) return launch_jk_coop(a, cw.coop_args, cw.coop_lds[mixed], mixed, (int)cw.items.size(), sh, st);
     return launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, mixed, a, (int)cw.items.size(), sh, st);
 }
@@ -1341,7 +1352,7 @@ int hfg::check_private_segments(hfg_ctx* c, bool grad) {
     const bool mixed = c->opt.precision == HFG_MIXED;
     for (const ClassWork& cw : c->classes) {
         // the cooperative and Rys kernels hold their tables in LDS
-        if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop) continue;
+        if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop || jk_on_rys(c, cw, mixed)) continue;
         if ((grad ? grad_uses_coop(cw.la, cw.lb, cw.lc, cw.ld) : jk_uses_coop(cw.la, cw.lb, cw.lc, cw.ld)))
             return fail(c, HFG_ERR_UNSUPPORTED, "the class needs the cooperative kernel, whose LDS does not fit a "
                                                 "workgroup on this device");
@@ -1663,8 +1674,9 @@ int hfg_autotune(hfg_ctx* c, int what) {
         for (size_t k = 0; k < c->classes.size(); ++k) {
             ClassWork& cw = c->classes[k];
             bool& use_coop = grad ? cw.gcoop : cw.coop;
-            // a class on the Rys gradient kernel only has its grid to choose (fixed workgroup size)
-            const bool rys = grad && grad_on_rys(c, cw, c->opt.precision == HFG_MIXED);
+            // a class on a Rys kernel only has its grid to choose (fixed workgroup size)
+            const bool mixed = c->opt.precision == HFG_MIXED;
+            const bool rys = grad ? grad_on_rys(c, cw, mixed) : jk_on_rys(c, cw, mixed);
             const bool coop_ok = !rys && (grad ? cw.gcoop_ok : cw.coop_ok);
             const bool reg_ok = !rys && cw.la + cw.lb + cw.lc + cw.ld < kCoopRequiredL;
             LaunchShape& shape = grad ? cw.grad_shape : cw.jk_shape;
@@ -1826,15 +1838,18 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
     // vector's zeroing on the context's stream
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     for (size_t k = 0; k < c->classes.size(); ++k) {
-        // the FP64 per-lane kernel of the class, or its cooperative kernel where the J/K builds run
-        // that one (the per-shell items: a class on the shell-group lists has them too)
+        // the kernel that the class's FP64 J/K builds run (on the per-shell items: a class on the
+        // shell-group lists has them too)
         const ClassWork& cw = c->classes[k];
         JkArgs b = a;
         b.items = c->d_items.p + cw.dev_off;
         b.queue = c->d_queue.p + k;
         const int n_items = (int)cw.items.size();
         HFG_CHECK(c, launch_zero_ints(b.queue, 1, c->heavy));
-        if (cw.coop)
+        if (jk_on_rys(c, cw, false)) {
+            const RysJkArgs ra{b, c->rys, nullptr, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
+            HFG_CHECK(c, launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, ra, n_items, LaunchShape{0, 0}, c->heavy));
+        } else if (cw.coop)
             HFG_CHECK(c, launch_jk_coop(b, cw.coop_args, cw.coop_lds[0], 0, n_items, LaunchShape{0, 0}, c->heavy));
         else
             HFG_CHECK(c, launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, 0, b, n_items, LaunchShape{0, 0}, c->heavy));

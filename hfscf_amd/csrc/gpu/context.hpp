@@ -145,9 +145,9 @@ struct hfg_ctx {
     // the device's shared stream for kernels that may spill to scratch (see shared_scratch_stream)
     hipStream_t heavy = nullptr;
     hipEvent_t ev_heavy_join = nullptr;
-    std::vector<int> class_stream;  // side stream of each class's J/K launch (-1: the shared stream)
-    std::vector<int> grad_stream[2];  // the same for the gradient launches, FP64 and mixed
-    std::vector<int> class_order, grad_order[2];  // launch order of the classes (J/K, gradient)
+    std::vector<int> class_stream[2];  // side stream of each class's J/K launch, FP64 and mixed (-1: the shared stream)
+    std::vector<int> grad_stream[2];   // the same for the gradient launches
+    std::vector<int> class_order[2], grad_order[2];  // launch order of the classes (J/K, gradient)
     // hardware queue of each side stream and of the shared stream (equal values: one queue, whose
     // kernels run one after another); the stream balance spreads the classes over the queues
     int side_queue[hfg::kSideStreams] = {};
@@ -269,6 +269,8 @@ namespace hfg {
 // Two-electron gradients (concatenated natom x 3 per molecule) through the adjoint
 // derivative kernels, for the concatenated densities D.
 int run_gradient(hfg_ctx* c, const double* D, double* grad);
+// d_Dc from the device densities D, enqueued on st (what the FP64 Rys kernels read).
+int make_cart_density(hfg_ctx* c, const double* D, hipStream_t st);
 }  // namespace hfg
 
 namespace hfg {
@@ -279,9 +281,9 @@ namespace hfg {
 // a J/K build that is captured in a graph), or only those on the shared stream.
 enum class ClassSet { All, Side, Shared };
 
-// Streams of the class launches (J/K, or the gradient in the context's precision when grad).
+// Streams of the class launches (J/K, or the gradient when grad) in the context's precision.
 inline const std::vector<int>& class_streams(const hfg_ctx* c, bool grad) {
-    return grad ? c->grad_stream[c->opt.precision == HFG_MIXED ? 1 : 0] : c->class_stream;
+    return (grad ? c->grad_stream : c->class_stream)[c->opt.precision == HFG_MIXED ? 1 : 0];
 }
 
 // Number of classes that run on the shared stream (J/K, or the gradient when grad). Their
@@ -308,7 +310,7 @@ inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn
     if (shared && (e = hipStreamWaitEvent(c->heavy, c->ev_fork, 0)) != hipSuccess) return e;
     // the shared-stream classes first: they are few workgroups of long latency, and launched
     // after the side streams' persistent grids they would wait for compute units to drain
-    const std::vector<int>& order = grad ? c->grad_order[c->opt.precision == HFG_MIXED ? 1 : 0] : c->class_order;
+    const std::vector<int>& order = (grad ? c->grad_order : c->class_order)[c->opt.precision == HFG_MIXED ? 1 : 0];
     int q = 0;
     for (int pass = 0; pass < 2; ++pass)
         for (size_t n = 0; n < c->classes.size(); ++n) {
@@ -338,12 +340,33 @@ constexpr int kGradConcurrentBytes = 4096;
 
 // Whether the FP64 gradient of a class runs the Rys kernel (rys_grad.hpp): from L = 4, where the
 // register kernels spill (2.7 KB per lane at (pp|pp) to 13 KB at (dd|pp), all slower: (pp|pp) of
-// (H2O)16 44 ms against 28, of water 2.8 ms against 0.06) and the program kernel, from L = 7, works
-// on one primitive quartet at a time; a context that asks for the program kernels (coop_min_l)
-// keeps them.
+// (H2O)16 25 ms alone against 16, of water 2.7 ms against 0.06) and the program kernel, from L = 7,
+// works on one primitive quartet at a time. The four L = 4 classes with a d shell hardly spill,
+// and with lanes to fill the register kernel is faster; measured alone on (H2O)n / cc-pVDZ, register
+// / Rys in ms, the lines lie where the two meet:
+//   (dp|ps) n = 4 1.8 / 1.5, 6 2.1 / 2.8, 16 18 / 36;   (ds|pp) n = 8 3.5 / 2.9, 12 5.7 / 7.4, 16 13 / 20;
+//   (ds|ds) n = 6 0.96 / 0.86, 8 1.13 / 1.12, 16 4.1 / 7;   (dd|ss) n = 1 0.23 / 0.04, 4 0.63 / 0.77.
+// A context that asks for the program kernels (coop_min_l) keeps them.
 inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
-    return !mixed && l >= kRysGradMinL && (c->opt.coop_min_l == 0 || l < c->opt.coop_min_l);
+    if (mixed || l < kRysGradMinL || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    if (!grad_keeps_register(cw.la, cw.lb, cw.lc, cw.ld)) return true;
+    const long long most = cw.lb == 2 ? 2500 : cw.lb == 1 ? 50000 : cw.lc == 2 ? 100000 : 400000;
+    return cw.quartets <= most;
+}
+
+// Whether the FP64 J/K of a class runs the Rys kernel (rys_jk.hpp): from L = 6, where the register
+// kernels spill most (measured alone on (H2O)16, register / Rys in ms: (dp|dp) 3.8 / 1.1, (dd|pp) 2.4 /
+// 0.67, (dd|dp) 1.35 / 0.33, (dp|dd) 0.63 / 0.13, (dd|dd) 0.53 / 0.09, (ds|dd) 0.54 / 0.21, (dd|ds)
+// 0.59 / 0.49), and for L = 4 and 5 only with few shell quartets, whose primitives it spreads over
+// lanes (water's (pp|pp) 0.15 / 0.04; (H2O)16 0.76 / 6, (dp|ps) 1.0 / 19): at about 10 ns per shell
+// quartet it meets the register kernels' 0.05 to 0.1 ms of latency near kRysJkFew. A context that
+// asks for the program kernels (coop_min_l) keeps them.
+constexpr long long kRysJkFew = 5000;
+inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
+    const int l = cw.la + cw.lb + cw.lc + cw.ld;
+    if (mixed || l < kRysJkSmallL || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    return l >= kRysJkMinL || cw.quartets <= kRysJkFew;
 }
 
 // Whether a class launch runs on the device's shared stream (one kernel at a time): J/K register
@@ -351,7 +374,7 @@ inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
 // segment in this build is above kGradConcurrentBytes (the scratch bound decides where the table
 // has no entry).
 inline bool on_shared_stream(const hfg_ctx* c, const ClassWork& cw, bool grad, bool mixed) {
-    if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop) return false;
+    if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop || jk_on_rys(c, cw, mixed)) return false;
     if (!grad) return class_spills(cw.la, cw.lb, cw.lc, cw.ld, false);
     const int b = private_segment_bytes(true, mixed, cw.la, cw.lb, cw.lc, cw.ld, c->pure);
     return b < 0 ? class_spills(cw.la, cw.lb, cw.lc, cw.ld, true) : b > kGradConcurrentBytes;

@@ -63,16 +63,16 @@ hipError_t launch_grad_any(hfg_ctx* c, const ClassWork& cw, const GradArgs& b, L
     return launch_grad(cw.la, cw.lb, cw.lc, cw.ld, c->pure, mixed, b, (int)cw.items.size(), sh, st);
 }
 
-// The Cartesian densities of the Rys kernels from d_D (a Cartesian basis reads d_D itself).
-int make_cart_density(hfg_ctx* c, hipStream_t st) {
+}  // namespace
+
+// The Cartesian densities of the Rys kernels from the densities D on the device (a Cartesian basis
+// reads D itself; the mixed kernels read none).
+int make_cart_density(hfg_ctx* c, const double* D, hipStream_t st) {
     if (c->opt.precision == HFG_MIXED || !c->pure) return HFG_OK;
-    HFG_CHECK(c, c->d_Dc.ensure(c->nc_total));
-    HFG_CHECK(c, launch_to_cart(c->d_D.p, c->d_mols.p, c->d_mol_cart.p, (int)c->mols.size(), c->max_ncart,
-                                c->d_cart_terms.p, c->d_Dc.p, st));
+    HFG_CHECK(c, launch_to_cart(D, c->d_mols.p, c->d_mol_cart.p, (int)c->mols.size(), c->max_ncart, c->d_cart_terms.p,
+                                c->d_Dc.p, st));
     return HFG_OK;
 }
-
-}  // namespace
 
 int run_gradient(hfg_ctx* c, const double* D, double* grad) {
     if (int r = check_private_segments(c, true)) return r;
@@ -90,7 +90,7 @@ int run_gradient(hfg_ctx* c, const double* D, double* grad) {
     GradArgs a = grad_args(c);
     const int mixed = c->opt.precision == HFG_MIXED ? 1 : 0;
     HFG_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    if (int r = make_cart_density(c, c->stream)) return r;
+    if (int r = make_cart_density(c, c->d_D.p, c->stream)) return r;
     HFG_CHECK(c, launch_zero_ints(c->d_queue.p + ncls, ncls, c->stream));
     HFG_CHECK(c, for_each_class_concurrent(c, c->stream, [&](const ClassWork& cw, hipStream_t st, int qi) {
         GradArgs b = a;
@@ -126,8 +126,7 @@ int run_one_class(hfg_ctx* c, size_t k, bool grad, LaunchShape sh) {
     hipStream_t st = class_launch_stream(c, k, grad);
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     HFG_CHECK(c, launch_zero_ints(q, 1, st));
-    if (grad)
-        if (int r = make_cart_density(c, st)) return r;
+    if (int r = make_cart_density(c, c->d_D.p, st)) return r;
     HFG_CHECK(c, hipEventRecord(c->ev0, st));
     if (grad) {
         HFG_CHECK(c, c->d_grad_slab.ensure((size_t)std::max<long long>(c->grad_slab_doubles, 1)));

@@ -17,14 +17,14 @@ HFG_FOR_CLASSES(HFG_DECL)
 
 namespace {
 
-// The register kernels: FP64 below L = kRysGradMinL (from there the context launches the Rys
-// kernel), mixed below L = 7 (from there it launches the cooperative kernel, coop_grad.hpp).
+// The register kernels: FP64 below L = 4 and for the L = 4 classes with a d shell (the context launches
+// the Rys kernel for the others), mixed below L = 7 (from there it launches the cooperative kernel, coop_grad.hpp).
 template <int A, int B, int C, int D, bool P>
 hipError_t grad_class(const GradArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
     const LaunchShape bs = scratch_safe_shape(A, B, C, D, true, sh, nitems);
     if constexpr (!grad_uses_coop(A, B, C, D))
         if (mixed) return launch_grad_class32<A, B, C, D, P>(a, nitems, bs, s);
-    if constexpr (A + B + C + D < kRysGradMinL)
+    if constexpr (grad_keeps_register(A, B, C, D))
         if (!mixed) return launch_grad_class64<A, B, C, D, P>(a, nitems, bs, s);
     return hipErrorInvalidValue;
 }

@@ -1,9 +1,10 @@
 // Run-time dispatch from (la lb|lc ld), basis type and precision to the specialised J/K kernel.
-// The classes from L = 7 up run the wavefront-cooperative kernel (coop.hpp), launched by the
-// context, and have no register kernel.
+// The context launches the others itself: the Rys kernel (rys_jk.hpp; FP64 from L = 6) and the
+// wavefront-cooperative kernel (coop.hpp; mixed from L = 7).
 #include "coop_args.hpp"
 #include "jk_impl.hpp"
 #include "launch_bounds.hpp"
+#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -21,11 +22,11 @@ namespace {
 
 template <int A, int B, int C, int D, bool P>
 hipError_t jk_class(const JkArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
-    if constexpr (A + B + C + D >= 7) {
-        return hipErrorInvalidValue;
-    } else {
-        return mixed ? launch_jk_class32<A, B, C, D, P>(a, nitems, sh, s) : launch_jk_class64<A, B, C, D, P>(a, nitems, sh, s);
-    }
+    if constexpr (A + B + C + D < 7)
+        if (mixed) return launch_jk_class32<A, B, C, D, P>(a, nitems, sh, s);
+    if constexpr (A + B + C + D < kRysJkMinL)
+        if (!mixed) return launch_jk_class64<A, B, C, D, P>(a, nitems, sh, s);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace

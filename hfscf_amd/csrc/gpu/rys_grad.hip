@@ -1,5 +1,6 @@
-// Run-time dispatch of the Rys gradient kernels and the Cartesian densities that they read.
+// Run-time dispatch of the Rys gradient and J/K kernels and the Cartesian densities that they read.
 #include "rys_grad.hpp"
+#include "rys_jk.hpp"
 
 namespace hfg {
 
@@ -19,6 +20,24 @@ hipError_t launch_rys_grad(int la, int lb, int lc, int ld, const RysGradArgs& a,
     RysGradArgs b = a;
     b.g.nitems = nitems;
     HFG_FOR_CLASSES(HFG_RYS_CASE)
+    return hipErrorInvalidValue;
+}
+
+#define HFG_DECL(A, B, C, D) \
+    template <>              \
+    hipError_t launch_rys_jk_class<A, B, C, D>(const RysJkArgs&, LaunchShape, hipStream_t);
+HFG_FOR_CLASSES(HFG_DECL)
+#undef HFG_DECL
+
+#define HFG_RYS_JK_CASE(A, B, C, D)   \
+    if constexpr (jk_has_rys(A, B, C, D)) \
+        if (la == A && lb == B && lc == C && ld == D) return launch_rys_jk_class<A, B, C, D>(b, sh, s);
+
+hipError_t launch_rys_jk(int la, int lb, int lc, int ld, const RysJkArgs& a, int nitems, LaunchShape sh, hipStream_t s) {
+    if (nitems == 0) return hipSuccess;
+    RysJkArgs b = a;
+    b.j.nitems = nitems;
+    HFG_FOR_CLASSES(HFG_RYS_JK_CASE)
     return hipErrorInvalidValue;
 }
 

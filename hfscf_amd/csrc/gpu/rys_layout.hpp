@@ -4,6 +4,13 @@
 namespace hfg {
 
 constexpr int kRysGradMinL = 4;    // FP64 gradient classes from this L run the Rys kernel
+// FP64 J/K classes from kRysJkMinL run the Rys kernel, from kRysJkSmallL those with few shell quartets.
+constexpr int kRysJkMinL = 6, kRysJkSmallL = 4;
+constexpr bool jk_has_rys(int la, int lb, int lc, int ld) { return la + lb + lc + ld >= kRysJkSmallL; }
+// Gradient classes that keep their FP64 register kernel for many shell quartets.
+constexpr bool grad_keeps_register(int la, int lb, int lc, int ld) {
+    return la + lb + lc + ld < kRysGradMinL || (la + lb + lc + ld == 4 && la == 2);
+}
 constexpr int kRysMaxN = 6;        // rules of 1..6 points (degree 11: total order up to 11)
 constexpr int kRysDeg = 9;         // polynomial degree per interval
 constexpr int kRysPerUnit = 2;     // intervals per unit of T
