@@ -1140,7 +1140,7 @@ int enqueue_classes(hfg_ctx* c, hipStream_t main, bool dscreen, bool timed, Clas
     a.dmax = c->d_dmax.p;
     a.dtol = dscreen ? c->opt.density_tol : 0.0;
     if (set != ClassSet::Shared)
-        if (int r = hfg::make_cart_density(c, buf.D, main)) return r;
+        if (int r = hfg::make_cart_density(c, buf.D, false, main)) return r;
     const int ncls = (int)c->classes.size(), nshared = shared_class_count(c, false);
     if (set != ClassSet::Shared) HFG_CHECK(c, launch_zero_ints(buf.queue + nshared, ncls - nshared, main));
     bool shared_zeroed = false;

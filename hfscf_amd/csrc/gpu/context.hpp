@@ -52,8 +52,9 @@ constexpr int kSideStreams = 8;  // most side streams a context may use (hfg_opt
 // 43.8/25.8, 34.3/18.0, 33.6/18.9, 34.6/18.9, 33.4/17.6 ms; (H2O)8 15.8/11.0, 10.1/6.3, 9.2/5.6,
 // 10.8/6.4, 8.9/5.5 ms.
 constexpr int kDefaultSideStreams = 6;
-// Classes from L = la+lb+lc+ld = kCoopRequiredL have only the cooperative kernels; from
-// kCoopTuneMinL up both forms exist and hfg_options.coop_min_l / hfg_autotune choose.
+// Classes from L = la+lb+lc+ld = kCoopRequiredL have no register kernel: they run the Rys kernels, or
+// the cooperative ones when hfg_options.coop_min_l asks for them. From kCoopTuneMinL up a class that
+// is not on a Rys kernel has both forms, and coop_min_l / hfg_autotune choose.
 constexpr int kCoopRequiredL = 7;
 constexpr int kCoopTuneMinL = 4;
 // Autotuning tries the cooperative form from this L only: below it the per-lane register kernels
@@ -269,8 +270,9 @@ namespace hfg {
 // Two-electron gradients (concatenated natom x 3 per molecule) through the adjoint
 // derivative kernels, for the concatenated densities D.
 int run_gradient(hfg_ctx* c, const double* D, double* grad);
-// d_Dc from the device densities D, enqueued on st (what the FP64 Rys kernels read).
-int make_cart_density(hfg_ctx* c, const double* D, hipStream_t st);
+// d_Dc from the device densities D, enqueued on st, when a class of the J/K build (or of the gradient
+// when grad) runs a Rys kernel, which reads it.
+int make_cart_density(hfg_ctx* c, const double* D, bool grad, hipStream_t st);
 }  // namespace hfg
 
 namespace hfg {
@@ -338,7 +340,7 @@ inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn
 // there in every build.
 constexpr int kGradConcurrentBytes = 4096;
 
-// Whether the FP64 gradient of a class runs the Rys kernel (rys_grad.hpp): from L = 4, where the
+// Whether the gradient of a class runs the Rys kernel (rys_grad.hpp): from L = 4, where the
 // register kernels spill (2.7 KB per lane at (pp|pp) to 13 KB at (dd|pp), all slower: (pp|pp) of
 // (H2O)16 25 ms alone against 16, of water 2.7 ms against 0.06) and the program kernel, from L = 7,
 // works on one primitive quartet at a time. The four L = 4 classes with a d shell hardly spill,
@@ -346,26 +348,31 @@ constexpr int kGradConcurrentBytes = 4096;
 // / Rys in ms, the lines lie where the two meet:
 //   (dp|ps) n = 4 1.8 / 1.5, 6 2.1 / 2.8, 16 18 / 36;   (ds|pp) n = 8 3.5 / 2.9, 12 5.7 / 7.4, 16 13 / 20;
 //   (ds|ds) n = 6 0.96 / 0.86, 8 1.13 / 1.12, 16 4.1 / 7;   (dd|ss) n = 1 0.23 / 0.04, 4 0.63 / 0.77.
-// A context that asks for the program kernels (coop_min_l) keeps them.
+// A mixed gradient runs it from L = 7, as the J/K build does ((H2O)8 32 -> 26 ms, (H2O)16 91 -> 82). A
+// context that asks for the program kernels (coop_min_l) keeps them.
 inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
-    if (mixed || l < kRysGradMinL || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    if (l < (mixed ? kRysMixedL : kRysGradMinL) || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
     if (!grad_keeps_register(cw.la, cw.lb, cw.lc, cw.ld)) return true;
     const long long most = cw.lb == 2 ? 2500 : cw.lb == 1 ? 50000 : cw.lc == 2 ? 100000 : 400000;
     return cw.quartets <= most;
 }
 
-// Whether the FP64 J/K of a class runs the Rys kernel (rys_jk.hpp): from L = 6, where the register
+// Whether the J/K of a class runs the Rys kernel (rys_jk.hpp): from L = 6, where the register
 // kernels spill most (measured alone on (H2O)16, register / Rys in ms: (dp|dp) 3.8 / 1.1, (dd|pp) 2.4 /
 // 0.67, (dd|dp) 1.35 / 0.33, (dp|dd) 0.63 / 0.13, (dd|dd) 0.53 / 0.09, (ds|dd) 0.54 / 0.21, (dd|ds)
 // 0.59 / 0.49), and for L = 4 and 5 only with few shell quartets, whose primitives it spreads over
 // lanes (water's (pp|pp) 0.15 / 0.04; (H2O)16 0.76 / 6, (dp|ps) 1.0 / 19): at about 10 ns per shell
-// quartet it meets the register kernels' 0.05 to 0.1 ms of latency near kRysJkFew. A context that
-// asks for the program kernels (coop_min_l) keeps them.
+// quartet it meets the register kernels' 0.05 to 0.1 ms of latency near kRysJkFew. A mixed build
+// runs it, in FP64, from L = 7, where its other kernel is the FP32 program kernel, one quartet at a time
+// (per build, program / Rys in ms: (dd|dp), (dp|dd), (dd|dd) of (H2O)8 1.28 / 0.17, 0.49 / 0.08, 0.56 /
+// 0.09, of (H2O)16 1.45 / 0.34, 0.67 / 0.13, 0.56 / 0.09; whole builds 4.35 -> 3.89, 17.9 -> 17.2); below, the
+// FP32 register kernels win ((dp|dp) of (H2O)16 0.62 against 1.06). A context that asks for the program
+// kernels (coop_min_l) keeps them.
 constexpr long long kRysJkFew = 5000;
 inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
-    if (mixed || l < kRysJkSmallL || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    if (l < (mixed ? kRysMixedL : kRysJkSmallL) || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
     return l >= kRysJkMinL || cw.quartets <= kRysJkFew;
 }
 

@@ -1,5 +1,6 @@
 // Two-electron RHF gradient driver (adjoint derivative-ERI kernels) and the single-class runs
 // of the launch-shape autotuner.
+#include <algorithm>
 #include <vector>
 
 #include "context.hpp"
@@ -66,9 +67,13 @@ hipError_t launch_grad_any(hfg_ctx* c, const ClassWork& cw, const GradArgs& b, L
 }  // namespace
 
 // The Cartesian densities of the Rys kernels from the densities D on the device (a Cartesian basis
-// reads D itself; the mixed kernels read none).
-int make_cart_density(hfg_ctx* c, const double* D, hipStream_t st) {
-    if (c->opt.precision == HFG_MIXED || !c->pure) return HFG_OK;
+// reads D itself).
+int make_cart_density(hfg_ctx* c, const double* D, bool grad, hipStream_t st) {
+    const bool mixed = c->opt.precision == HFG_MIXED;
+    const bool read = std::any_of(c->classes.begin(), c->classes.end(), [&](const ClassWork& cw) {
+        return grad ? grad_on_rys(c, cw, mixed) : jk_on_rys(c, cw, mixed);
+    });
+    if (!c->pure || !read) return HFG_OK;
     HFG_CHECK(c, launch_to_cart(D, c->d_mols.p, c->d_mol_cart.p, (int)c->mols.size(), c->max_ncart, c->d_cart_terms.p,
                                 c->d_Dc.p, st));
     return HFG_OK;
@@ -90,7 +95,7 @@ int run_gradient(hfg_ctx* c, const double* D, double* grad) {
     GradArgs a = grad_args(c);
     const int mixed = c->opt.precision == HFG_MIXED ? 1 : 0;
     HFG_CHECK(c, hipEventRecord(c->ev0, c->stream));
-    if (int r = make_cart_density(c, c->d_D.p, c->stream)) return r;
+    if (int r = make_cart_density(c, c->d_D.p, true, c->stream)) return r;
     HFG_CHECK(c, launch_zero_ints(c->d_queue.p + ncls, ncls, c->stream));
     HFG_CHECK(c, for_each_class_concurrent(c, c->stream, [&](const ClassWork& cw, hipStream_t st, int qi) {
         GradArgs b = a;
@@ -126,7 +131,7 @@ int run_one_class(hfg_ctx* c, size_t k, bool grad, LaunchShape sh) {
     hipStream_t st = class_launch_stream(c, k, grad);
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     HFG_CHECK(c, launch_zero_ints(q, 1, st));
-    if (int r = make_cart_density(c, c->d_D.p, st)) return r;
+    if (int r = make_cart_density(c, c->d_D.p, grad, st)) return r;
     HFG_CHECK(c, hipEventRecord(c->ev0, st));
     if (grad) {
         HFG_CHECK(c, c->d_grad_slab.ensure((size_t)std::max<long long>(c->grad_slab_doubles, 1)));

@@ -18,7 +18,8 @@ HFG_FOR_CLASSES(HFG_DECL)
 namespace {
 
 // The register kernels: FP64 below L = 4 and for the L = 4 classes with a d shell (the context launches
-// the Rys kernel for the others), mixed below L = 7 (from there it launches the cooperative kernel, coop_grad.hpp).
+// the Rys kernel for the others), mixed below L = 7 (from there it launches the Rys kernel too, or on
+// request the cooperative one, coop_grad.hpp).
 template <int A, int B, int C, int D, bool P>
 hipError_t grad_class(const GradArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
     const LaunchShape bs = scratch_safe_shape(A, B, C, D, true, sh, nitems);

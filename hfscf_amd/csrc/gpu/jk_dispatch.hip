@@ -1,6 +1,6 @@
 // Run-time dispatch from (la lb|lc ld), basis type and precision to the specialised J/K kernel.
-// The context launches the others itself: the Rys kernel (rys_jk.hpp; FP64 from L = 6) and the
-// wavefront-cooperative kernel (coop.hpp; mixed from L = 7).
+// The context launches the others itself: the Rys kernel (rys_jk.hpp; FP64 from L = 6, mixed from 7) and the
+// wavefront-cooperative kernel (coop.hpp; on request).
 #include "coop_args.hpp"
 #include "jk_impl.hpp"
 #include "launch_bounds.hpp"

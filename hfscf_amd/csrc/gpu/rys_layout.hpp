@@ -6,6 +6,8 @@ namespace hfg {
 constexpr int kRysGradMinL = 4;    // FP64 gradient classes from this L run the Rys kernel
 // FP64 J/K classes from kRysJkMinL run the Rys kernel, from kRysJkSmallL those with few shell quartets.
 constexpr int kRysJkMinL = 6, kRysJkSmallL = 4;
+// Mixed builds and gradients run the same FP64 kernels from kRysMixedL.
+constexpr int kRysMixedL = 7;
 constexpr bool jk_has_rys(int la, int lb, int lc, int ld) { return la + lb + lc + ld >= kRysJkSmallL; }
 // Gradient classes that keep their FP64 register kernel for many shell quartets.
 constexpr bool grad_keeps_register(int la, int lb, int lc, int ld) {

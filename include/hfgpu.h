@@ -62,10 +62,12 @@ typedef struct hfg_options {
     int work_split;       /* work items per class launch relative to the default split (1, 2, 4, ...;
                              0 = the default). More items keep more wavefronts in flight at the cost of
                              more tiles to gather. */
-    int coop_min_l;       /* classes with la+lb+lc+ld >= coop_min_l run on the wavefront-cooperative
-                             kernels (one workgroup per quartet, recursion tables in LDS), the others
-                             on the per-lane register kernels; 4..7, 0 = 7 (the default). From L = 4 up,
-                             hfg_autotune keeps whichever form it measures faster for each class. */
+    int coop_min_l;       /* 4..7: classes with la+lb+lc+ld >= coop_min_l run on the wavefront-cooperative
+                             kernels (one workgroup per quartet, recursion tables in LDS). 0 = the default:
+                             the Rys kernels where they are faster (FP64 J/K from L = 6 and gradients from
+                             L = 4, mixed from L = 7, and L = 4 and 5 of small molecules), the per-lane
+                             register kernels elsewhere, where hfg_autotune tries the cooperative form
+                             too and keeps what it measures faster for each class. */
     int side_streams;     /* streams the class launches of one build are spread over (1..8, 0 = 6) */
     int group_shells;     /* 0 or 1 (the default): s shells of one atom with identical exponents (the
                              contracted s shells of cc-pVXZ, which share one set of primitives) form

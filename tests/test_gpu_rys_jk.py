@@ -2,7 +2,7 @@
 their branches change: Cartesian and spherical d, with and without the screen (element screen and
 Cartesian diagonal), one centre (T = 0), a dimer 40 bohr apart (T beyond the table), the
 density-screened incremental build, and a batch on both sides of the shell-quartet count that moves
-L = 4 and 5 between the kernels. The exported ERI vector has the same integrals.
+L = 4 and 5 between the kernels, and mixed contexts from L = 7. The exported ERI vector has the same integrals.
 
 Tolerance: 1e-11 on J and K (integrals good to a few 1e-15 summed over at most 48^2 densities of
 about 0.1) and 1e-12 on single integrals."""
@@ -69,3 +69,20 @@ def test_rys_jk_batch_across_the_quartet_count():
     n = mols[0].nbf
     for got, ref in zip((J, K), one):
         assert np.abs(got.reshape(len(mols), n, n) - ref).max() < 1e-11
+
+
+@pytest.mark.parametrize("basis", ["6-31g**", "cc-pvdz"])
+@pytest.mark.parametrize("kind", ["water", "near", "far"])
+def test_mixed_runs_fp64_rys_from_l7(kind, basis):
+    # a density over the d functions alone: J and K between them come from (dd|dd) only, and so does the
+    # gradient's two-electron part; a mixed context has both to FP64
+    mol = H.Molecule.from_arrays(*_system(kind), basis)
+    s = mol.shells()
+    d = np.concatenate([np.arange(o, o + (5 if mol.pure else 6))
+                        for L, o in zip(s["L"], s["pure_off"] if mol.pure else s["cart_off"]) if L == 2])
+    D = np.zeros((mol.nbf, mol.nbf))
+    D[np.ix_(d, d)] = _density(len(d), 7)
+    ctx, ref = H.GpuContext(mol, precision=H.MIXED), H.GpuContext(mol)
+    for got, want in zip(ctx.build_jk(D), ref.build_jk(D)):
+        assert np.abs(got - want)[np.ix_(d, d)].max() < 1e-11
+    assert np.abs(ctx.energy_backward(D) - ref.energy_backward(D)).max() < 1e-11
