@@ -16,6 +16,7 @@
 #include "coop.hpp"
 #include "coop_grad.hpp"
 #include "flopmodel.hpp"
+#include "host_copy.hpp"
 #include "launch_bounds.hpp"
 #include "misc.hpp"
 #include "noalloc.hpp"
@@ -1834,29 +1835,30 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
     a.dmax = c->d_dmax.p;
     a.dtol = 0.0;
     a.eri_out = c->d_eri_out.p;
-    // the class kernels may spill: they run on the device's shared scratch stream, after the
-    // vector's zeroing on the context's stream
+    // after the vector's zeroing the classes run as in an FP64 build, in its launch order and over its
+    // streams ((H2O)8 / cc-pVDZ: 16 ms of kernels one after another, 8 ms so)
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
-    for (size_t k = 0; k < c->classes.size(); ++k) {
+    for (int k : c->class_order[0]) {
         // the kernel that the class's FP64 J/K builds run (on the per-shell items: a class on the
         // shell-group lists has them too)
         const ClassWork& cw = c->classes[k];
+        hipStream_t st = on_shared_stream(c, cw, false, false) ? c->heavy : c->side[std::max(c->class_stream[0][k], 0)];
         JkArgs b = a;
         b.items = c->d_items.p + cw.dev_off;
         b.queue = c->d_queue.p + k;
         const int n_items = (int)cw.items.size();
-        HFG_CHECK(c, launch_zero_ints(b.queue, 1, c->heavy));
+        HFG_CHECK(c, launch_zero_ints(b.queue, 1, st));
         if (jk_on_rys(c, cw, false)) {
             const RysJkArgs ra{b, c->rys, nullptr, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
-            HFG_CHECK(c, launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, ra, n_items, LaunchShape{0, 0}, c->heavy));
+            HFG_CHECK(c, launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, ra, n_items, LaunchShape{0, 0}, st));
         } else if (cw.coop)
-            HFG_CHECK(c, launch_jk_coop(b, cw.coop_args, cw.coop_lds[0], 0, n_items, LaunchShape{0, 0}, c->heavy));
+            HFG_CHECK(c, launch_jk_coop(b, cw.coop_args, cw.coop_lds[0], 0, n_items, LaunchShape{0, 0}, st));
         else
-            HFG_CHECK(c, launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, 0, b, n_items, LaunchShape{0, 0}, c->heavy));
+            HFG_CHECK(c, launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, 0, b, n_items, LaunchShape{0, 0}, st));
     }
     HFG_CHECK(c, hipStreamSynchronize(c->heavy));
-    HFG_CHECK(c, hipMemcpyAsync(out, c->d_eri_out.p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HFG_CHECK(c, hipStreamSynchronize(c->stream));
+    for (int k = 0; k < c->nside; ++k) HFG_CHECK(c, hipStreamSynchronize(c->side[k]));
+    HFG_CHECK(c, copy_to_host(out, c->d_eri_out.p, (size_t)n * sizeof(double), c->device, c->stream));
     c->d_eri_out.release();  // the vector grows as N^4; the context keeps no copy
     return HFG_OK;
 }
