@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "boys.hpp"
+#include "boys_lds.hpp"
 #include "context.hpp"
 #include "coop.hpp"
 #include "coop_grad.hpp"
@@ -1865,7 +1866,8 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
 
 int hfg_boys_probe(hfg_ctx* c, int m, int n, const double* T, double* F, int closed_form) {
     if (!c) return HFG_ERR_ARG;
-    if (!T || !F || n < 0 || m < 0 || m > kBoysMaxM || (closed_form && m > 1))
+    if (!T || !F || n < 0 || m < 0 || m > kBoysMaxM ||
+        (closed_form == 2 ? m > kBoysLdsMaxM : closed_form && m > 1))
         return fail(c, HFG_ERR_ARG, "hfg_boys_probe: bad arguments");
     for (int i = 0; i < n; ++i)
         if (!(T[i] >= 0.0)) return fail(c, HFG_ERR_ARG, "hfg_boys_probe: T must be >= 0");

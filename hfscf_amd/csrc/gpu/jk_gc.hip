@@ -2,9 +2,11 @@
 // identical exponents (cc-pVDZ oxygen has two s shells on the same nine exponents) share their
 // primitive pairs, so each primitive quartet of a group quartet is evaluated once (prefactor,
 // Boys value) and contracted into every member shell quartet with that member's coefficients.
-// Every member quartet then gets what the per-shell kernel gives it: hfscf's primitive cutoff on
-// its own prefactor, the mean-Schwarz shell skip and the density screen on its own pairs, the
-// element screen, the Cartesian diagonal from the screen matrix, and its digestion.
+// A primitive quartet is dropped when the prefactor of every member is below hfscf's cutoff. The sum
+// over the ket primitives runs per ket member only; the bra members' coefficients multiply it once
+// per bra primitive. Every member quartet then gets what the per-shell kernel gives it: the
+// mean-Schwarz shell skip and the density screen on its own pairs, the element screen, the Cartesian
+// diagonal from the screen matrix, and its digestion.
 // A group quartet of many primitive quartets (two 9-primitive groups: 6561) would hold one lane
 // for as long as its members take on many lanes of the per-shell kernel, so the work item's
 // `split` lanes share it, each over a slice of the bra primitive pairs; each lane digests its
@@ -13,22 +15,26 @@
 #include <type_traits>
 
 #include "boys32.hpp"
+#include "boys_lds.hpp"
 #include "gc.hpp"
 #include "jk_gc_impl.hpp"
 #include "jk_impl.hpp"
 
 namespace hfg {
 
-// Three wavefronts per SIMD: the FP64 kernel then holds 168 VGPRs and keeps 84 bytes per lane in
-// scratch, against 185 VGPRs and two wavefronts without the attribute; alone on the (H2O)16 /
-// cc-pVDZ build it took 5.0 ms instead of 5.9 (the FP32 kernel fits four wavefronts either way).
-// The FP64 (ps|ss) group kernel, forced the same way, spilled 340 bytes per lane and slowed from
-// 8.1 to 11.4 ms.
+// Bound: latency at three wavefronts per SIMD (168 VGPRs, 68 bytes of scratch per lane), which forcing
+// them buys. Alone on the (H2O)16 / cc-pVDZ build, FP64: 5.03 ms with every member's product in the
+// inner loop, 4.79 with the ket summed first, 3.27 with the Boys table in LDS, 2.98 with the next ket
+// primitive's exponent and centre loaded ahead (with its coefficients too the kernel spills and takes
+// longer); the FP32 kernel of the mixed builds 3.05 -> 2.63.
 template <typename R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void jk_gc_ssss_kernel(JkArgs a, GcArgs g) {
     __shared__ double tiles[kRegions * kBlockFuncs * kBlockFuncs];
     __shared__ int rowpre[kMaxRows + 1];
     __shared__ int next_item;
+    constexpr bool lds_boys = std::is_same_v<R, double>;
+    __shared__ __align__(16) double boys[lds_boys ? boys_lds_size(0) : 2];
+    if constexpr (lds_boys) boys_lds_load<0>(a.boys, boys);
     const bool dscreen = a.dtol > 0.0;
     const R cut = (R)a.prim_cut;
     R jab[kGcMaxShells * kGcMaxShells];  // J_ab partials of the current bra row, per member
@@ -109,9 +115,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void j
                 const double4 Kb = g.gK[gb.off + ib * gb.pstride];
                 const R Kbm[4] = {(R)Kb.x, (R)Kb.y, (R)Kb.z, (R)Kb.w};
                 const R kbmax = fmax(fmax(fabs(Kbm[0]), fabs(Kbm[1])), fmax(fabs(Kbm[2]), fabs(Kbm[3])));
+                R part[kGcMaxMembers] = {(R)0, (R)0, (R)0, (R)0};  // this bra primitive's sums over the ket, per ket member
+                int icn = gk.off;
+                double4 nb0 = g.gp0[icn];
                 for (int jk = 0; jk < gk.np; ++jk) {
-                    const double4 b0 = g.gp0[gk.off + jk * gk.pstride];
-                    const double4 Kk = g.gK[gk.off + jk * gk.pstride];
+                    const int ic = icn;
+                    const double4 b0 = nb0, Kk = g.gK[ic];
+                    icn += jk + 1 < gk.np ? gk.pstride : 0;  // stays in bounds on the last primitive
+                    nb0 = g.gp0[icn];
                     const R Kkm[4] = {(R)Kk.x, (R)Kk.y, (R)Kk.z, (R)Kk.w};
                     const R kkmax = fmax(fmax(fabs(Kkm[0]), fabs(Kkm[1])), fmax(fabs(Kkm[2]), fabs(Kkm[3])));
                     R rs, F0[1];
@@ -137,20 +148,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void j
                         double T = a0.x * b0.x * ipq * r2;
                         // hfscf floors T at 1e-8 inside F_nu and uses F_0 = 1 when r_PQ^2 <= 1e-18
                         T = (r2 > 1e-18) ? fmax(T, 1e-8) : 0.0;
-                        boys_low<0, double>(T, 1.0, F0);
+                        boys_lds<0>(T, boys, 1.0, F0);
                     }
+                    const R v = rs * F0[0];
 #pragma unroll
-                    for (int mb = 0; mb < kGcMaxMembers; ++mb) {
-                        if (mb >= gb.nmem) continue;
-                        const R kb = Kbm[mb];
+                    for (int mk = 0; mk < kGcMaxMembers; ++mk)
+                        if (mk < gk.nmem) part[mk] += Kkm[mk] * v;
+                }
 #pragma unroll
-                        for (int mk = 0; mk < kGcMaxMembers; ++mk) {
-                            if (mk >= gk.nmem) continue;
-                            R pfac = kb * Kkm[mk] * rs;
-                            pfac = (fabs(pfac) < cut) ? (R)0 : pfac;
-                            acc[mb][mk] += pfac * F0[0];
-                        }
-                    }
+                for (int mb = 0; mb < kGcMaxMembers; ++mb) {
+                    if (mb >= gb.nmem) continue;
+#pragma unroll
+                    for (int mk = 0; mk < kGcMaxMembers; ++mk) acc[mb][mk] += Kbm[mb] * part[mk];
                 }
             }
             // the member quartets, one at a time (the loops stay rolled: one copy of the digestion;

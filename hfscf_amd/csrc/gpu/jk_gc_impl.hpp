@@ -4,9 +4,10 @@
 // A pair of an s group and a shell (or of two s groups) has up to gc_members member shell pairs
 // that share every primitive pair (exponents, centres, 1/2p, P - A) and differ only in K. Each
 // primitive quartet of a group quartet gets one prefactor, one set of Boys values (scaled by
-// 1/sqrt(p + q) alone) and one vertical recursion, whose results are added into every member
-// quartet's accumulators with that member's K_ab K_cd, after hfscf's primitive cutoff on the
-// member's own prefactor K_ab K_cd / sqrt(p + q). Each member quartet is then finished as the
+// 1/sqrt(p + q) alone) and one vertical recursion, whose results are summed over the ket primitives
+// with each ket member's K_cd, and once per bra primitive with each bra member's K_ab into the member
+// quartets' accumulators. A primitive quartet is dropped when the prefactor K_ab K_cd / sqrt(p + q) of
+// every member is below hfscf's cutoff. Each member quartet is then finished as the
 // per-shell kernel finishes a quartet: horizontal recursion, element screen, spherical transform
 // or Cartesian diagonal, and digestion, after the mean-Schwarz and density screens on its own
 // pairs. As in the (ss|ss) group kernel, a work item's `split` lanes share each group quartet over
@@ -15,17 +16,20 @@
 #include <type_traits>
 
 #include "boys32.hpp"
+#include "boys_lds.hpp"
 #include "gc.hpp"
 #include "jk_impl.hpp"
 
 namespace hfg {
 
-// The FP32 kernel of the mixed builds at four wavefronts per SIMD (128 VGPRs and 60 bytes of
-// scratch per lane for (ps|ss), against 162 VGPRs and three wavefronts unconstrained); the FP64
-// kernel unconstrained (forced to three wavefronts it kept 340 bytes per lane in scratch and
-// slowed from 8.1 to 11.4 ms on the (H2O)16 build).
+// The FP32 kernel of the mixed builds at four wavefronts per SIMD (128 VGPRs and 100 bytes of
+// scratch per lane for (ps|ss), against 162 VGPRs and three wavefronts unconstrained), the FP64
+// kernel at two (forced to three it kept 340 bytes per lane in scratch and slowed from 8.1 to 11.4 ms
+// on the (H2O)16 build; with one, at 262 VGPRs, 11.2). FP64 (ps|ss) alone there: 8.03 ms with every
+// member's product in the inner loop, 7.18 with the ket summed first, 5.86 with the Boys table in LDS,
+// 5.76 with the next ket primitive's exponent and centre loaded ahead; FP32 4.57 -> 4.13.
 template <int LA, int LB, int LC, int LD, bool PURE, typename R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same_v<R, float> ? 4 : 1))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(std::is_same_v<R, float> ? 4 : 2))) void
 jk_gc_kernel(JkArgs a, GcArgs g) {
     constexpr int LT = LA + LB + LC + LD;
     static_assert(LT > 0, "(ss|ss) has its own group kernel");
@@ -39,6 +43,9 @@ jk_gc_kernel(JkArgs a, GcArgs g) {
     __shared__ double tiles[kRegions * kBlockFuncs * kBlockFuncs];
     __shared__ int rowpre[kMaxRows + 1];
     __shared__ int next_item;
+    constexpr bool lds_boys = std::is_same_v<R, double>;
+    __shared__ __align__(16) double boys[lds_boys ? boys_lds_size(LT) : 2];
+    if constexpr (lds_boys) boys_lds_load<LT>(a.boys, boys);
     const bool dscreen = a.dtol > 0.0;
     R jab[MB][NA * NB];  // J_ab partials of the current bra row, per member
     int jab_o[MB];
@@ -129,9 +136,17 @@ jk_gc_kernel(JkArgs a, GcArgs g) {
                     Kbm[m] = (R)Kbd[m];
                     kbmax = fmax(kbmax, fabs(Kbm[m]));
                 });
+                R part[MK][H::NE][H::NF];  // this bra primitive's sums over the ket, per ket member
+                sfor<MK>([&](auto y) {
+                    sfor<H::NE>([&](auto e) { sfor<H::NF>([&](auto f) { part[y][e][f] = (R)0; }); });
+                });
+                int icn = gk.off;
+                double4 nb0 = g.gp0[icn];
                 for (int jk = 0; jk < gk.np; ++jk) {
-                    const int ic = gk.off + jk * gk.pstride;
-                    const double4 b0 = g.gp0[ic];
+                    const int ic = icn;
+                    const double4 b0 = nb0;
+                    icn += jk + 1 < gk.np ? gk.pstride : 0;  // stays in bounds on the last primitive
+                    nb0 = g.gp0[icn];
                     const double4 b1 = g.gp1[ic];
                     const double4 Kk = g.gK[ic];
                     const double Kkd[4] = {Kk.x, Kk.y, Kk.z, Kk.w};
@@ -171,10 +186,7 @@ jk_gc_kernel(JkArgs a, GcArgs g) {
                         const double ipq = rs * rs;
                         const double T = p * q * ipq * r2;
                         double F[LT + 1];
-                        if constexpr (LT == 1)
-                            boys_low<1, double>(T, rs, F);
-                        else
-                            boys_eval_rs<LT, double>(T, a.boys, rs, F);
+                        boys_lds<LT>(T, boys, rs, F);
                         const double rp = q * ipq, rq = p * ipq;
                         const double PA[3] = {a1.x, a1.y, a1.z};
                         const double QC[3] = {b1.x, b1.y, b1.z};
@@ -182,21 +194,21 @@ jk_gc_kernel(JkArgs a, GcArgs g) {
                         const double WQ[3] = {rq * PQx, rq * PQy, rq * PQz};
                         V.run(F, PA, WP, QC, WQ, a1.w, rp, b1.w, rq, 0.5 * ipq);
                     }
-                    sfor<MB>([&](auto x) {
-                        if (x < gb.nmem)
-                            sfor<MK>([&](auto y) {
-                                if (y < gk.nmem) {
-                                    const R kk = Kbm[x] * Kkm[y];
-                                    const R wgt = (fabs(kk * rs) < (R)a.prim_cut) ? (R)0 : kk;
-                                    sfor<H::NE>([&](auto e) {
-                                        sfor<H::NF>([&](auto f) {
-                                            acc[x][y][e][f] += wgt * V.v[H::NE0 + e][H::NF0 + f][0];
-                                        });
-                                    });
-                                }
+                    sfor<MK>([&](auto y) {
+                        if (y < gk.nmem)
+                            sfor<H::NE>([&](auto e) {
+                                sfor<H::NF>([&](auto f) { part[y][e][f] += Kkm[y] * V.v[H::NE0 + e][H::NF0 + f][0]; });
                             });
                     });
                 }
+                sfor<MB>([&](auto x) {
+                    if (x < gb.nmem)
+                        sfor<MK>([&](auto y) {
+                            sfor<H::NE>([&](auto e) {
+                                sfor<H::NF>([&](auto f) { acc[x][y][e][f] += Kbm[x] * part[y][e][f]; });
+                            });
+                        });
+                });
             }
             // the member quartets, one at a time (rolled loops: one copy of the finishing code;
             // member indices come from memory, the accumulators through select chains, since

@@ -1,4 +1,5 @@
 // Schwarz diagonal, gather, counter reset and Fock kernels.
+#include "boys_lds.hpp"
 #include "jk_impl.hpp"
 #include "misc.hpp"
 
@@ -190,15 +191,28 @@ hipError_t launch_block_absmax(const double* D, const MolDev* mols, const int* s
 
 // ------------------------------------------------------------------ Boys probe (test hook)
 // F_0..F_M at n values of T through the device functions the class kernels use: the table
-// with Taylor step and recursions (boys_eval_rs), or the closed forms of F_0 and F_1 (boys_low).
+// with Taylor step and recursions (boys_eval_rs, form 0), the closed forms of F_0 and F_1 (boys_low, 1) or
+// the LDS table (boys_lds, 2).
 template <int M>
 __global__ void boys_probe_kernel(const double* __restrict__ T, const double* __restrict__ tab, double* out, int n,
-                                  int closed_form) {
+                                  int form) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if constexpr (M <= kBoysLdsMaxM) {
+        if (form == 2) {  // every lane of the workgroup reaches the barrier
+            __shared__ __align__(16) double lds[boys_lds_size(M)];
+            boys_lds_load<M>(tab, lds);
+            __syncthreads();
+            if (i >= n) return;
+            double F[M + 1];
+            boys_lds<M>(T[i], lds, 1.0, F);
+            for (int m = 0; m <= M; ++m) out[(size_t)i * (M + 1) + m] = F[m];
+            return;
+        }
+    }
     if (i >= n) return;
     double F[M + 1];
     if constexpr (M <= 1) {
-        if (closed_form) {
+        if (form) {
             boys_low<M, double>(T[i], 1.0, F);
         } else {
             boys_eval_rs<M, double>(T[i], tab, 1.0, F);
@@ -225,7 +239,7 @@ hipError_t launch_boys_probe_m(int m, const double* T, const double* tab, double
 hipError_t launch_boys_probe(int m, const double* T, const double* tab, double* out, int n, int closed_form,
                              hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    if (m < 0 || m > kBoysMaxM || (closed_form && m > 1)) return hipErrorInvalidValue;
+    if (m < 0 || m > kBoysMaxM || (closed_form == 2 ? m > kBoysLdsMaxM : closed_form && m > 1)) return hipErrorInvalidValue;
     return launch_boys_probe_m<0>(m, T, tab, out, n, closed_form, s);
 }
 

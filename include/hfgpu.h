@@ -156,7 +156,8 @@ int hfg_schwarz(hfg_ctx* ctx, double* screen);
 
 /* Test hook: F_0..F_m(T) (n x (m+1), row-major) for n values T >= 0, evaluated on the device by
  * the functions the class kernels use: the tabulated Taylor step with down/upward recursion
- * (closed_form = 0, m <= 17) or the closed forms of F_0 and F_1 (closed_form = 1, m <= 1).
+ * (closed_form = 0, m <= 17), the closed forms of F_0 and F_1 (closed_form = 1, m <= 1) or the
+ * Taylor sums over the table in LDS (closed_form = 2, m <= 4).
  * Replaces: extramath::F_nu and the downward recursion at its call site (hfscf: src/math/gamma.cpp:18-24,
  * src/integrals/hfscf_oseri.cpp:103-118), without hfscf's T >= 1e-8 floor, which the kernels apply
  * where hfscf does (L = 0 quartets). */
