@@ -10,7 +10,10 @@
 // the HRR to the six shifted classes and contracts them with G at once, so derivative
 // integrals are never stored.
 #pragma once
+#include <type_traits>
+
 #include "boys.hpp"
+#include "boys_lds.hpp"
 #include "common.hpp"
 #include "hgp.hpp"
 
@@ -140,10 +143,27 @@ HFG_INLINE void hrr_from_vrr(const Vrr<LAB1, LCD1, R>& V, const R* AB, const R* 
     H::run(acc, AB, CD, out);
 }
 
+// A shell quartet's primitive quartets are split over the lanes of a work item, over the bra pairs
+// first: so that a lane has at most about kGradLanePrims of them, and further, down to kGradMinPrims
+// (each slice builds the two-particle density and adds its sums to the atoms' again), while the item has
+// fewer than four slices per lane. One lane per quartet took 0.14 us per primitive quartet in series:
+// water / 6-31G* (ss|ss) 576 -> 12 us, (ps|ss) 375 -> 15, (pp|ps) 506 -> 43; its gradient 1.46 -> 0.34 ms.
+constexpr int kGradLanePrims = 512, kGradMinPrims = 8;
+
+// Wavefronts per SIMD that the registers of a kernel are held to (1 = no limit). Alone on (H2O)16 /
+// cc-pVDZ in ms, FP64: (ss|ss) 16.7 free, 15.3 at 3; (ps|ss) 20.5, 18.8 at 3; (ps|ps), 4 registers
+// above two wavefronts, 13.6, 11.8 at 2, 32 at 3; (pp|ss) 7.3, 5.8 at 2, 12 at 3; (ds|ss) 3.8, 3.9 at 2;
+// the larger ones spill at 2 ((pp|ps) 8.7, 28 at 2).
+constexpr int grad_waves(int la, int lb, int lc, int ld, bool fp64) {
+    const int l = la + lb + lc + ld;
+    return !fp64 ? 1 : l <= 1 ? 3 : l == 2 && la == 1 ? 2 : 1;
+}
+
 // R = double: FP64 throughout. R = float (mixed mode): two-particle density, VRR, HRR and
 // contraction in FP32; Boys values and pair data from FP64, per-item atom sums in FP64.
 template <int LA, int LB, int LC, int LD, bool PURE, typename R>
-__global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves(LA, LB, LC, LD, std::is_same_v<R, double>)))) void
+grad_kernel(GradArgs a) {
     constexpr int NA = PURE && LA > 0 ? 2 * LA + 1 : ncart(LA);
     constexpr int NB = PURE && LB > 0 ? 2 * LB + 1 : ncart(LB);
     constexpr int NC = PURE && LC > 0 ? 2 * LC + 1 : ncart(LC);
@@ -153,6 +173,9 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
     __shared__ double gsum[kMaxAtoms * 3];
     __shared__ int rowpre[kMaxRows + 1];
     __shared__ int next_item;
+    constexpr bool lds_boys = std::is_same_v<R, double> && LT + 1 <= kBoysLdsMaxM;
+    __shared__ __align__(16) double boys[lds_boys ? boys_lds_size(LT + 1) : 2];
+    if constexpr (lds_boys) boys_lds_load<LT + 1>(a.boys, boys);
     for (;;) {
     __syncthreads();  // the previous item's flush has read gsum and next_item
     if (threadIdx.x == 0) next_item = atomicAdd(a.queue, 1);
@@ -180,7 +203,12 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
     }
     __syncthreads();
     const int total = rowpre[nrows];
-    for (int t = threadIdx.x; t < total; t += blockDim.x) {
+    // the pairs of a block pair have one primitive count, so one split serves the item
+    const int nb = total > 0 ? a.pairs[bpo].np : 1, nk = total > 0 ? a.pairs[kpo].np : 1;
+    const int want = max(nb * nk / kGradLanePrims, min(nb * nk / kGradMinPrims, 4 * (int)blockDim.x / max(total, 1)));
+    const int sb = max(1, min(want, nb)), sk = max(1, min(want / sb, nk)), split = sb * sk;
+    for (int u = threadIdx.x; u < total * split; u += blockDim.x) {
+        const int slice = u / total, t = u - slice * total, slb = slice / sk, slk = slice - slb * sk;
         int lo = 0, hi = nrows;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -224,15 +252,18 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
         R gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
         const R AB[3] = {(R)bp.AB[0], (R)bp.AB[1], (R)bp.AB[2]};
         const R CD[3] = {(R)kp.AB[0], (R)kp.AB[1], (R)kp.AB[2]};
-        for (int ip = 0; ip < bp.np; ++ip) {
+        for (int ip = slb; ip < bp.np; ip += sb) {
             const int ia = bp.off + ip * bp.pstride;
             const double4 a0 = a.pp0[ia];
             const double4 a1 = a.pp1[ia];
             const double4 a2 = a.pp2[ia];
             const double p = a0.x;
-            for (int jp = 0; jp < kp.np; ++jp) {
+            constexpr bool ahead = lds_boys;  // load the next ket primitive's exponent and centre ahead
+            double4 nb0 = a.pp0[kp.off + min(slk, kp.np - 1) * kp.pstride];
+            for (int jp = slk; jp < kp.np; jp += sk) {
                 const int ib = kp.off + jp * kp.pstride;
-                const double4 b0 = a.pp0[ib];
+                const double4 b0 = ahead ? nb0 : a.pp0[ib];
+                if constexpr (ahead) nb0 = a.pp0[jp + sk < kp.np ? ib + sk * kp.pstride : ib];  // stays in bounds
                 const double4 b1 = a.pp1[ib];
                 const double4 b2 = a.pp2[ib];
                 const double q = b0.x;
@@ -244,7 +275,10 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
                 const double ipq = rs * rs;
                 const double T = p * q * ipq * r2;
                 R F[LT + 2];
-                boys_eval<LT + 1, R>(T, a.boys, pfac, F);
+                if constexpr (lds_boys)
+                    boys_lds<LT + 1>(T, boys, pfac, F);
+                else
+                    boys_eval<LT + 1, R>(T, a.boys, pfac, F);
                 const double rp = q * ipq, rq = p * ipq;
                 const R PA[3] = {(R)a1.x, (R)a1.y, (R)a1.z};
                 const R QC[3] = {(R)b1.x, (R)b1.y, (R)b1.z};

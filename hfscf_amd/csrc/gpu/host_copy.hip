@@ -3,10 +3,11 @@
 // One hipMemcpy into pages the caller has not touched yet is bound by one host thread that faults them
 // in and copies: 10 GB/s, where the link gives 52. Here up to kThreads host threads take chunks in turn; each
 // has the device write a chunk into one of its two pinned buffers while it copies the other one out, so that
-// the page faults and the copies of the threads run beside the link's transfers. Measured on the 1.6 GB
-// ERI vector of (H2O)8 / cc-pVDZ, fresh huge / small pages: one thread 117 / 349 ms, 2 61 / 214, 4 39 / 122,
+// the page faults and the copies of the threads run beside the link's transfers. Measured on 1.6 GB,
+// fresh huge / small pages: one thread 117 / 349 ms, 2 61 / 214, 4 39 / 122,
 // 8 35 / 71, 12 35 / 61; chunks of 1 MB 51 ms, 4 MB 35, 16 MB 31 but 88 on small pages. The buffers
-// (64 MB, 0.5 ms to allocate) live for the call only.
+// (64 MB, 0.5 ms to allocate) live for the call only. The 1.37 GB ERI vector of (H2O)8 / cc-pVDZ with
+// its kernels: 145 -> 41 ms.
 #include "host_copy.hpp"
 
 #include <algorithm>
