@@ -39,8 +39,19 @@ HFG_INLINE void export_block(const R* I, const PairDev& bp, const PairDev& kp, b
     });
 }
 
+// Wavefronts per SIMD that the registers of a kernel are held to (1 = no limit): two for the FP64 classes that
+// come out a few registers above the 256 of two ((pp|ps) 289, (ps|pp) 271, (dd|ss) 262). Alone on
+// (H2O)16 / cc-pVDZ in ms, free / at two: (pp|ps) 1.63 / 1.34, (ps|pp) 0.82 / 0.65, (dd|ss) 0.19 / 0.16.
+// The others lose: at two (pp|pp) 0.76 / 2.1, (dp|ps) 1.04 / 1.57, (ds|pp) 0.69 / 1.43; at three, from
+// 194 to 217 registers, (ps|ps) 3.75 / 3.89, (pp|ss) 1.84 / 2.05, (ds|ss) 1.6 / 1.67.
+constexpr int jk_waves(int la, int lb, int lc, int ld, bool fp64) {
+    const int l = la + lb + lc + ld;
+    return fp64 && ((l == 3 && la == 1) || (la == 2 && lb == 2 && l == 4)) ? 2 : 1;
+}
+
 template <int LA, int LB, int LC, int LD, bool PURE, typename R, typename ACC>
-__global__ __launch_bounds__(256) void jk_kernel(JkArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_waves(LA, LB, LC, LD, std::is_same_v<R, double>)))) void
+jk_kernel(JkArgs a) {
     constexpr int NA = PURE && LA > 0 ? 2 * LA + 1 : ncart(LA);
     constexpr int NB = PURE && LB > 0 ? 2 * LB + 1 : ncart(LB);
     constexpr int NC = PURE && LC > 0 ? 2 * LC + 1 : ncart(LC);
