@@ -712,7 +712,7 @@ int setup_geometry(hfg_ctx* c) {
                     const FlopParts fp = model_flops(cw.la, cw.lb, cw.lc, cw.ld, c->pure, false);
                     for (int i = 0; i < c->gcnt[P]; ++i) gc_cost[ci] += gc_row(P, Q, i, cw, fp).second;
                 }
-    const double split = c->opt.work_split > 0 ? (double)c->opt.work_split : kDefaultWorkSplit;
+    const double split = c->opt.work_split > 0 ? (double)c->opt.work_split : default_work_split(c->opt.schwarz != 0);
     const double target = std::max(total_cost / (256.0 * 6.0 * split), 1.0);
     c->slab_doubles = 0;
     c->grad_slab_doubles = 0;

@@ -110,11 +110,13 @@ struct MolHost {
     int gout0 = 0;               // offset of its natom x 3 gradient in concatenated output
 };
 
-// Default split of a class launch into work items (hfg_options.work_split replaces it): four times
-// the items of one per 1/1536 of the build's model cost, which keeps several wavefronts per SIMD
-// busy in the wide s and p classes (measured on (H2O)16 / cc-pVDZ: 48 ms per FP64 build at 1,
-// 37 at 2, 36 at 4, 38 at 8).
-constexpr double kDefaultWorkSplit = 4.0;
+// Default split of a class launch into work items (hfg_options.work_split replaces it), relative to one
+// item per 1/1536 of the build's model cost. More items keep more wavefronts in flight and cost more
+// tiles to flush and gather. FP64 builds with the screen at 1, 2, 4 in ms: (H2O)8 4.7, 5.0, 6.0, (H2O)16
+// 25.7, 25.4, 25.9, C12H26 / 6-31G** 4.8, 5.0, 5.5, 64 molecules 9.7, 10.0, 11.2; mixed (H2O)8 3.0, 3.1,
+// 3.8. The gradient has no tiles and wants more: (H2O)8 21.5, 19.5, 18.9, mixed (H2O)16 147, 120, 108.
+// A context without the screen is the gradient's (hfscf's visits every quartet), so the screen decides.
+constexpr double default_work_split(bool screened) { return screened ? 1.0 : 4.0; }
 
 // Cached graph of one J/K build configuration.
 struct JkGraph {

@@ -19,11 +19,10 @@
  *   - Status 0 = success, negative = error; hfg_last_error() gives the message. The library
  *     never exits the process and never falls back to a CPU path.
  *   - A context owns its main stream, its side streams (six by default) and all its device
- *     memory; it is not thread-safe. The class kernels that spill (private segments of several
- *     KB per lane) run on one more stream that every context on a device shares, one launch at
- *     a time, so that a single queue holds their scratch (hfg_eri_vector and hfg_hessian_2e
- *     launch there too); contexts used from several threads on
- *     one device therefore serialise those launches, and a HIP graph (hfg_options.graph) never
+ *     memory; it is not thread-safe. The class kernels that spill most (private segments of several
+ *     KB per lane: mixed gradient classes) run on one more stream that every context on a device
+ *     shares, one launch at a time, so that a single queue holds their scratch; contexts used from
+ *     several threads on one device therefore serialise those launches, and a HIP graph (hfg_options.graph) never
  *     captures them (they are launched directly at each replay).
  */
 #ifndef HFGPU_H
@@ -60,7 +59,8 @@ typedef struct hfg_options {
                              hfscf_hf_solver.cpp:317-324); 0 = off (default) */
     int graph;            /* 1 = capture each J/K build configuration once as a HIP graph and replay it */
     int work_split;       /* work items per class launch relative to the default split (1, 2, 4, ...;
-                             0 = the default). More items keep more wavefronts in flight at the cost of
+                             0 = the default, 1 with the Schwarz screen and 4
+                             without). More items keep more wavefronts in flight at the cost of
                              more tiles to gather. */
     int coop_min_l;       /* 4..7: classes with la+lb+lc+ld >= coop_min_l run on the wavefront-cooperative
                              kernels (one workgroup per quartet, recursion tables in LDS). 0 = the default:
