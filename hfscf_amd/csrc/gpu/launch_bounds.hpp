@@ -15,11 +15,11 @@ inline size_t class_scratch_bound(int la, int lb, int lc, int ld, bool grad) {
     return sizeof(double) * (size_t)vrr_entries(lab, lcd, lt);
 }
 
-// Classes whose kernels run on the device's shared stream, one at a time. Gradient: every class
-// whose bound exceeds kSpillBytes (the register kernels of the d classes spill 10-13 KB per
-// lane; the workspace kernels share one workspace per context). J/K: the classes whose bound
-// exceeds kJkSharedBytes, (dd|dd), (dd|dp) and (dp|dd), which spill 9-14 KB per lane; the
-// other J/K classes spill at most 4.3 KB per lane and run concurrently on the side streams.
+// Classes whose register kernels run on the device's shared stream, one at a time. Gradient: every
+// class whose bound exceeds kSpillBytes, where the build's table has no figure. J/K: the classes
+// whose bound exceeds kJkSharedBytes, (dd|dd), (dd|dp) and (dp|dd), which have no register kernel
+// any more; the others spill at most 1.2 KB per lane (FP64 (dp|pp); mixed (dd|pp) 0.9) and run concurrently
+// on the side streams.
 // (Per-lane private sizes as read from the code-object metadata of the built kernels.)
 constexpr size_t kSpillBytes = 2048;
 constexpr size_t kJkSharedBytes = 15000;

@@ -18,8 +18,7 @@
 //
 // Bound: FP64 VALU of R_tuv (the Boys step and the recursion). Measured per call, with the host's
 // copies: (H2O)16 / cc-pVDZ S, T, V 0.54 ms (3.2 with one lane per pair and nucleus on tables in
-// scratch); (H2O)8 / cc-pVDZ gradient terms 0.27 ms
-// (7.9).
+// scratch); (H2O)8 / cc-pVDZ gradient terms 0.27 ms (7.9).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -25,8 +25,8 @@ extern const int kNumPrivateSegments;
 
 constexpr int kMaxPrivateBytes = 13744;
 
-// Bytes per lane of the kernel a class launch runs (the mixed (dd|dd) gradient runs the FP64
-// workspace kernel); -1 when the table has no entry.
+// Bytes per lane of a class's register kernel (the FP64 one where no mixed kernel is built); -1 when the
+// table has no entry.
 inline int private_segment_bytes(bool grad, bool mixed, int la, int lb, int lc, int ld, bool pure) {
     for (int pass = 0; pass < 2; ++pass) {
         const int m = (pass == 0 && mixed) ? 1 : 0;
