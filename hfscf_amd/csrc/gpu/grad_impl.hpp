@@ -203,7 +203,7 @@ grad_kernel(GradArgs a) {
     }
     __syncthreads();
     const int total = rowpre[nrows];
-    // the pairs of a block pair have one primitive count, so one split serves the item
+    // one split for the item, by its lists' strongest pairs (a pair of more primitives has longer slices)
     const int nb = total > 0 ? a.pairs[bpo].np : 1, nk = total > 0 ? a.pairs[kpo].np : 1;
     const int want = max(nb * nk / kGradLanePrims, min(nb * nk / kGradMinPrims, 4 * (int)blockDim.x / max(total, 1)));
     const int sb = max(1, min(want, nb)), sk = max(1, min(want / sb, nk)), split = sb * sk;
