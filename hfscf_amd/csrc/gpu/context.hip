@@ -633,13 +633,18 @@ int setup_geometry(hfg_ctx* c) {
     }
     // work items per class
     std::vector<double> cum_np(c->pairs.size() + nbp, 0.0);  // per block pair prefix of np
+    std::vector<int> max_np(cum_np.size(), 0);               // and largest np of the prefix
     std::vector<int> cum_off(nbp, 0);
     {
         int k = 0;
         for (int P = 0; P < nbp; ++P) {
             cum_off[P] = k;
             cum_np[k++] = 0;
-            for (int i = 0; i < c->bp_cnt[P]; ++i, ++k) cum_np[k] = cum_np[k - 1] + c->pairs[c->bp_off[P] + i].np;
+            for (int i = 0; i < c->bp_cnt[P]; ++i, ++k) {
+                const int np = c->pairs[c->bp_off[P] + i].np;
+                cum_np[k] = cum_np[k - 1] + np;
+                max_np[k] = std::max(max_np[k - 1], np);
+            }
         }
     }
     for (auto& cw : c->classes) {
@@ -750,6 +755,7 @@ int setup_geometry(hfg_ctx* c) {
         }
         flush(nrows);
     };
+    std::vector<int> row_kets;  // ket pairs of each row of the bra list in hand
     for (int m = 0; m < (int)c->mols.size(); ++m) {
         const MolHost& M = c->mols[m];
         for (int P = M.bp0; P < M.bp0 + M.nbp; ++P)
@@ -778,7 +784,13 @@ int setup_geometry(hfg_ctx* c) {
                 w.C = C;
                 w.D = D;
                 w.mol = m;
+                row_kets.assign(c->bp_cnt[P], 0);
                 auto push = [&](int r0, int r1, int c0, int c1) {
+                    double prims = 0.0;
+                    for (int r = r0; r < r1; ++r)
+                        prims += c->pairs[c->bp_off[P] + r].np * (cum_np[cum_off[Q] + std::min(row_kets[r], c1)] -
+                                                                  cum_np[cum_off[Q] + std::min(row_kets[r], c0)]);
+                    cw.longest_item = std::max(cw.longest_item, prims);
                     WorkItem v = w;
                     v.r0 = r0;
                     v.r1 = r1;
@@ -795,6 +807,8 @@ int setup_geometry(hfg_ctx* c) {
                     if (P == Q) cnt = std::min(cnt, i + 1);
                     const double np_i = c->pairs[c->bp_off[P] + i].np;
                     const double kq = np_i * cum_np[cum_off[Q] + cnt];
+                    row_kets[i] = cnt;
+                    cw.heaviest_quartet = std::max(cw.heaviest_quartet, np_i * max_np[cum_off[Q] + cnt]);
                     cw.quartets += cnt;
                     cw.flops += kq * fp.per_prim + cnt * fp.per_quartet;
                     cw.grad_flops += kq * gp.per_prim + cnt * gp.per_quartet;

@@ -70,6 +70,7 @@ struct ClassWork {
     std::vector<WorkItem> items;
     size_t dev_off = 0;
     long long quartets = 0;
+    double longest_item = 0, heaviest_quartet = 0;  // primitive quartets of the longest item, the heaviest shell quartet
     double flops = 0;
     double grad_flops = 0;
     LaunchShape jk_shape{0, 0};    // persistent workgroups / block of the J/K launch (0 = automatic)
@@ -363,19 +364,37 @@ inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
 // Whether the J/K of a class runs the Rys kernel (rys_jk.hpp): from L = 6, where the register
 // kernels spill most (measured alone on (H2O)16, register / Rys in ms: (dp|dp) 3.8 / 1.1, (dd|pp) 2.4 /
 // 0.67, (dd|dp) 1.35 / 0.33, (dp|dd) 0.63 / 0.13, (dd|dd) 0.53 / 0.09, (ds|dd) 0.54 / 0.21, (dd|ds)
-// 0.59 / 0.49), and for L = 4 and 5 only with few shell quartets, whose primitives it spreads over
-// lanes (water's (pp|pp) 0.15 / 0.04; (H2O)16 0.76 / 6, (dp|ps) 1.0 / 19): at about 10 ns per shell
-// quartet it meets the register kernels' 0.05 to 0.1 ms of latency near kRysJkFew. A mixed build
-// runs it, in FP64, from L = 7, where its other kernel is the FP32 program kernel, one quartet at a time
-// (per build, program / Rys in ms: (dd|dp), (dp|dd), (dd|dd) of (H2O)8 1.28 / 0.17, 0.49 / 0.08, 0.56 /
-// 0.09, of (H2O)16 1.45 / 0.34, 0.67 / 0.13, 0.56 / 0.09; whole builds 4.35 -> 3.89, 17.9 -> 17.2); below, the
-// FP32 register kernels win ((dp|dp) of (H2O)16 0.62 against 1.06). A context that asks for the program
-// kernels (coop_min_l) keeps them.
+// 0.59 / 0.49), and for L = 4 and 5 only in small molecules. There both kernels are one serial chain: a
+// register lane runs its shell quartet's primitive quartets, a Rys workgroup those of its whole work
+// item, at rys_jk_item_limit times the lane's speed. So a class runs Rys while its longest item is within
+// that many of its heaviest shell quartet (and, beyond latency, while it has at most kRysJkFew shell
+// quartets, at about 10 ns each: (H2O)16 (pp|pp) 0.76 / 6, (dp|ps) 1.0 / 19). The limits lie where the
+// two meet; in ms in water clusters and alkanes of 1 to 6 heavy atoms, items as multiples of the heaviest quartet:
+//   (pp|pp) at 1: 0.147 / 0.043, 4: 0.161 / 0.144, 5: 0.157 / 0.164, 7: 0.181 / 0.222, 10: 0.20 / 0.30
+//   (ds|pp) 1: 0.073 / 0.028, 3: 0.213 / 0.145, 4: 0.087 / 0.093, 6: 0.084 / 0.145
+//   (ds|ds) 1: 0.044 / 0.029, 2: 0.096 / 0.070, 2.3: 0.046 / 0.064, 4: 0.050 / 0.099
+//   (dp|ps) 1.5: 0.056 / 0.046, 2: 0.137 / 0.102, 2.5: 0.138 / 0.148, 4: 0.073 / 0.109
+//   (dd|ss) 1.5: 0.039 / 0.044, 3: 0.075 / 0.100
+//   (dp|pp) 1: 0.183 / 0.027, 6: 0.191 / 0.118, 9: 0.184 / 0.153, 12: 0.250 / 0.261
+//   (ds|dp) 5: 0.098 / 0.082, 6: 0.099 / 0.093, 7: 0.098 / 0.108, 10: 0.194 / 0.226
+//   (dp|ds) 1.5: 0.088 / 0.039, 6: 0.109 / 0.115, 8: 0.102 / 0.150
+//   (dd|ps) 1.5: 0.062 / 0.039, 2: 0.100 / 0.062, 2.5: 0.094 / 0.100, 4: 0.063 / 0.089
+// (In STO-3G, whose p shells have three primitives, builds ran Rys on long items: C4H10 0.65 -> 0.54 ms, (H2O)5 0.63 -> 0.54.)
+// A mixed build runs it, in FP64, from L = 7, where its other kernel is the FP32 program kernel, one
+// quartet at a time (per build, program / Rys in ms: (dd|dp), (dp|dd), (dd|dd) of (H2O)8 1.28 / 0.17,
+// 0.49 / 0.08, 0.56 / 0.09, of (H2O)16 1.45 / 0.34, 0.67 / 0.13, 0.56 / 0.09; whole builds 4.35 -> 3.89,
+// 17.9 -> 17.2); below, the FP32 register kernels win ((dp|dp) of (H2O)16 0.62 against 1.06). A context
+// that asks for the program kernels (coop_min_l) keeps them.
 constexpr long long kRysJkFew = 5000;
+constexpr double rys_jk_item_limit(int la, int lb, int lc, int ld) {
+    if (la + lb + lc + ld == 4) return la == 1 ? 5.0 : lb == 2 ? 1.0 : lb == 1 || lc == 2 ? 2.0 : 3.0;
+    return lb == 2 ? 2.0 : lb == 0 ? 6.0 : lc == 2 ? 5.0 : 9.0;
+}
 inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
     if (l < (mixed ? kRysMixedL : kRysJkSmallL) || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
-    return l >= kRysJkMinL || cw.quartets <= kRysJkFew;
+    return l >= kRysJkMinL ||
+           (cw.quartets <= kRysJkFew && cw.longest_item <= rys_jk_item_limit(cw.la, cw.lb, cw.lc, cw.ld) * cw.heaviest_quartet);
 }
 
 // Whether a class launch runs on the device's shared stream (one kernel at a time): J/K register
