@@ -62,7 +62,7 @@ void assign_streams(hfg_ctx* c, bool grad, bool mixed, const std::vector<double>
     std::iota(ord.begin(), ord.end(), 0);
     auto coop = [&](size_t k) {
         const ClassWork& cw = c->classes[k];
-        return grad ? cw.gcoop && !grad_on_rys(c, cw, mixed) : cw.coop && !jk_on_rys(c, cw, mixed);
+        return grad ? cw.gcoop[mixed] && !grad_on_rys(c, cw, mixed) : cw.coop[mixed] && !jk_on_rys(c, cw, mixed);
     };
     std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) {
         if (coop(x) != coop(y)) return coop(x);
@@ -866,7 +866,7 @@ int setup_geometry(hfg_ctx* c) {
         std::vector<std::pair<size_t, CoopHostProgram>> progs;
         for (size_t k = 0; k < c->classes.size(); ++k) {
             ClassWork& cw = c->classes[k];
-            cw.coop = cw.coop_ok = false;
+            cw.coop[0] = cw.coop[1] = cw.coop_ok = false;
             if (class_l(cw) < kCoopTuneMinL) continue;
             CoopHostProgram hp = make_coop_program(cw.la, cw.lb, cw.lc, cw.ld, c->pure);
             cw.coop_lds[0] = hp.lds_bytes(false);
@@ -876,14 +876,14 @@ int setup_geometry(hfg_ctx* c) {
             words.insert(words.end(), hp.words.begin(), hp.words.end());
             progs.emplace_back(base, std::move(hp));
             cw.coop_ok = true;
-            cw.coop = class_l(cw) >= coop_min || jk_uses_coop(cw.la, cw.lb, cw.lc, cw.ld);
+            cw.coop[0] = cw.coop[1] = class_l(cw) >= coop_min || jk_uses_coop(cw.la, cw.lb, cw.lc, cw.ld);
         }
         // gradient programs of the same classes for the cooperative gradient kernel
         std::vector<int4> gwords;
         std::vector<std::pair<size_t, CoopGradHostProgram>> gprogs;
         for (size_t k = 0; k < c->classes.size(); ++k) {
             ClassWork& cw = c->classes[k];
-            cw.gcoop = cw.gcoop_ok = false;
+            cw.gcoop[0] = cw.gcoop[1] = cw.gcoop_ok = false;
             if (class_l(cw) < kCoopTuneMinL) continue;
             const size_t limit = (size_t)c->max_lds - kCoopGradStaticLds;
             CoopGradHostProgram hp;
@@ -898,7 +898,7 @@ int setup_geometry(hfg_ctx* c) {
             gwords.insert(gwords.end(), hp.words.begin(), hp.words.end());
             gprogs.emplace_back(base, std::move(hp));
             cw.gcoop_ok = true;
-            cw.gcoop = class_l(cw) >= coop_min || grad_uses_coop(cw.la, cw.lb, cw.lc, cw.ld);
+            cw.gcoop[0] = cw.gcoop[1] = class_l(cw) >= coop_min || grad_uses_coop(cw.la, cw.lb, cw.lc, cw.ld);
         }
         if (!gwords.empty()) {
             HFG_CHECK(c, c->d_gcoop.upload(gwords, c->stream));
@@ -1360,7 +1360,7 @@ hipError_t hfg::launch_jk_class(hfg_ctx* c, const ClassWork& cw, const JkArgs& a
         const RysJkArgs r{a, c->rys, c->pure ? c->d_Dc.p : a.D, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
         return launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, r, (int)cw.items.size(), sh, st);
     }
-    if (cw.coop) return launch_jk_coop(a, cw.coop_args, cw.coop_lds[mixed], mixed, (int)cw.items.size(), sh, st);
+    if (cw.coop[mixed]) return launch_jk_coop(a, cw.coop_args, cw.coop_lds[mixed], mixed, (int)cw.items.size(), sh, st);
     return launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, mixed, a, (int)cw.items.size(), sh, st);
 }
 
@@ -1368,7 +1368,7 @@ int hfg::check_private_segments(hfg_ctx* c, bool grad) {
     const bool mixed = c->opt.precision == HFG_MIXED;
     for (const ClassWork& cw : c->classes) {
         // the cooperative and Rys kernels hold their tables in LDS
-        if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop || jk_on_rys(c, cw, mixed)) continue;
+        if (grad ? cw.gcoop[mixed] || grad_on_rys(c, cw, mixed) : cw.coop[mixed] || jk_on_rys(c, cw, mixed)) continue;
         if ((grad ? grad_uses_coop(cw.la, cw.lb, cw.lc, cw.ld) : jk_uses_coop(cw.la, cw.lb, cw.lc, cw.ld)))
             return fail(c, HFG_ERR_UNSUPPORTED, "the class needs the cooperative kernel, whose LDS does not fit a "
                                                 "workgroup on this device");
@@ -1689,21 +1689,26 @@ int hfg_autotune(hfg_ctx* c, int what) {
         std::vector<double> measured(c->classes.size(), 0.0);
         for (size_t k = 0; k < c->classes.size(); ++k) {
             ClassWork& cw = c->classes[k];
-            bool& use_coop = grad ? cw.gcoop : cw.coop;
-            // a class on a Rys kernel only has its grid to choose (fixed workgroup size)
             const bool mixed = c->opt.precision == HFG_MIXED;
+            bool& use_coop = grad ? cw.gcoop[mixed] : cw.coop[mixed];
+            const bool was_coop = use_coop;
+            // a class on a Rys kernel only has its grid to choose (fixed workgroup size)
             const bool rys = grad ? grad_on_rys(c, cw, mixed) : jk_on_rys(c, cw, mixed);
             const bool coop_ok = !rys && (grad ? cw.gcoop_ok : cw.coop_ok);
-            const bool reg_ok = !rys && cw.la + cw.lb + cw.lc + cw.ld < kCoopRequiredL;
+            const bool reg_ok = !rys && (grad ? grad_has_register(cw.la, cw.lb, cw.lc, cw.ld, mixed)
+                                              : jk_has_register(cw.la, cw.lb, cw.lc, cw.ld, mixed));
             LaunchShape& shape = grad ? cw.grad_shape : cw.jk_shape;
-            bool best_coop = use_coop;
+            bool best_coop = was_coop;
             LaunchShape best = shape;
             float best_ms = 1e30f;
             auto trial = [&](bool coop, LaunchShape sh) -> int {
                 use_coop = coop;
                 float total = 0.0f;
                 for (int rep = 0; rep < 2; ++rep) {
-                    if (int e = hfg::run_one_class(c, k, grad, sh)) return e;
+                    if (int e = hfg::run_one_class(c, k, grad, sh)) {
+                        use_coop = was_coop;  // the context keeps a form that runs
+                        return e;
+                    }
                     float ms = 0.0f;
                     HFG_CHECK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
                     if (rep > 0) total += ms;  // the first run warms caches and code
@@ -1738,14 +1743,14 @@ int hfg_autotune(hfg_ctx* c, int what) {
 int hfg_launch_shapes(const hfg_ctx* c, int cap, int* la_lb_lc_ld, int* jk_grid, int* jk_block, int* grad_grid,
                       int* grad_block) {
     if (!c) return HFG_ERR_ARG;
-    const int n = (int)c->classes.size();
+    const int n = (int)c->classes.size(), mixed = c->opt.precision == HFG_MIXED ? 1 : 0;
     for (int k = 0; k < n && k < cap; ++k) {
         const ClassWork& cw = c->classes[k];
         if (la_lb_lc_ld) la_lb_lc_ld[k] = cw.la * 1000 + cw.lb * 100 + cw.lc * 10 + cw.ld;
         if (jk_grid) jk_grid[k] = cw.jk_shape.grid;
-        if (jk_block) jk_block[k] = cw.gc ? -2 : cw.coop ? -1 : cw.jk_shape.block;
+        if (jk_block) jk_block[k] = cw.gc ? -2 : cw.coop[mixed] ? -1 : cw.jk_shape.block;
         if (grad_grid) grad_grid[k] = cw.grad_shape.grid;
-        if (grad_block) grad_block[k] = cw.gcoop ? -1 : cw.grad_shape.block;
+        if (grad_block) grad_block[k] = cw.gcoop[mixed] ? -1 : cw.grad_shape.block;
     }
     return n;
 }
@@ -1866,7 +1871,7 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
         if (jk_on_rys(c, cw, false)) {
             const RysJkArgs ra{b, c->rys, nullptr, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
             HFG_CHECK(c, launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, ra, n_items, LaunchShape{0, 0}, st));
-        } else if (cw.coop)
+        } else if (cw.coop[0])
             HFG_CHECK(c, launch_jk_coop(b, cw.coop_args, cw.coop_lds[0], 0, n_items, LaunchShape{0, 0}, st));
         else
             HFG_CHECK(c, launch_jk(cw.la, cw.lb, cw.lc, cw.ld, c->pure, 0, b, n_items, LaunchShape{0, 0}, st));

@@ -52,9 +52,9 @@ constexpr int kSideStreams = 8;  // most side streams a context may use (hfg_opt
 // 43.8/25.8, 34.3/18.0, 33.6/18.9, 34.6/18.9, 33.4/17.6 ms; (H2O)8 15.8/11.0, 10.1/6.3, 9.2/5.6,
 // 10.8/6.4, 8.9/5.5 ms.
 constexpr int kDefaultSideStreams = 6;
-// Classes from L = la+lb+lc+ld = kCoopRequiredL have no register kernel: they run the Rys kernels, or
-// the cooperative ones when hfg_options.coop_min_l asks for them. From kCoopTuneMinL up a class that
-// is not on a Rys kernel has both forms, and coop_min_l / hfg_autotune choose.
+// Classes from L = la+lb+lc+ld = kCoopRequiredL have no register kernel in either precision. The classes
+// from kCoopTuneMinL up have a cooperative kernel, which hfg_options.coop_min_l asks for; autotuning may
+// move a class between it and the register kernel (where one exists, jk_has_register).
 constexpr int kCoopRequiredL = 7;
 constexpr int kCoopTuneMinL = 4;
 // Autotuning tries the cooperative form from this L only: below it the per-lane register kernels
@@ -78,12 +78,12 @@ struct ClassWork {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;  // brackets of the last direct launch
     // J/K on the wavefront-cooperative kernel: its program (device pointers into the context's
     // d_coop buffer) and the LDS bytes of its FP64 and mixed launches
-    bool coop = false;
+    bool coop[2] = {false, false};  // FP64 and mixed
     bool coop_ok = false;  // a program exists (the class may move between the two kernel forms)
     CoopArgs coop_args{};
     size_t coop_lds[2] = {0, 0};
     // the gradient on the cooperative kernel (program in d_gcoop)
-    bool gcoop = false;
+    bool gcoop[2] = {false, false};
     bool gcoop_ok = false;
     CoopGradArgs gcoop_args{};
     size_t gcoop_lds[2] = {0, 0};
@@ -343,6 +343,12 @@ inline hipError_t for_each_class_concurrent(hfg_ctx* c, hipStream_t main, F&& fn
 // there in every build.
 constexpr int kGradConcurrentBytes = 4096;
 
+// Whether the context asks for the cooperative kernels of the classes of this L (from kCoopRequiredL also
+// when they do not fit, which the build refuses).
+inline bool asks_coop(const hfg_ctx* c, int l, bool fits) {
+    return c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l && (fits || l >= kCoopRequiredL);
+}
+
 // Whether the gradient of a class runs the Rys kernel (rys_grad.hpp): from L = 4, where the
 // register kernels spill (2.7 KB per lane at (pp|pp) to 13 KB at (dd|pp), all slower: (pp|pp) of
 // (H2O)16 25 ms alone against 16, of water 2.7 ms against 0.06) and the program kernel, from L = 7,
@@ -352,10 +358,10 @@ constexpr int kGradConcurrentBytes = 4096;
 //   (dp|ps) n = 4 1.8 / 1.5, 6 2.1 / 2.8, 16 18 / 36;   (ds|pp) n = 8 3.5 / 2.9, 12 5.7 / 7.4, 16 13 / 20;
 //   (ds|ds) n = 6 0.96 / 0.86, 8 1.13 / 1.12, 16 4.1 / 7;   (dd|ss) n = 1 0.23 / 0.04, 4 0.63 / 0.77.
 // A mixed gradient runs it from L = 7, as the J/K build does ((H2O)8 32 -> 26 ms, (H2O)16 91 -> 82). A
-// context that asks for the program kernels (coop_min_l) keeps them.
+// context that asks for the program kernels (coop_min_l) keeps them, where they fit.
 inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
-    if (l < (mixed ? kRysMixedL : kRysGradMinL) || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    if (l < (mixed ? kRysMixedL : kRysGradMinL) || asks_coop(c, l, cw.gcoop_ok)) return false;
     if (!grad_keeps_register(cw.la, cw.lb, cw.lc, cw.ld)) return true;
     const long long most = cw.lb == 2 ? 2500 : cw.lb == 1 ? 50000 : cw.lc == 2 ? 100000 : 400000;
     return cw.quartets <= most;
@@ -384,7 +390,7 @@ inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
 // quartet at a time (per build, program / Rys in ms: (dd|dp), (dp|dd), (dd|dd) of (H2O)8 1.28 / 0.17,
 // 0.49 / 0.08, 0.56 / 0.09, of (H2O)16 1.45 / 0.34, 0.67 / 0.13, 0.56 / 0.09; whole builds 4.35 -> 3.89,
 // 17.9 -> 17.2); below, the FP32 register kernels win ((dp|dp) of (H2O)16 0.62 against 1.06). A context
-// that asks for the program kernels (coop_min_l) keeps them.
+// that asks for the program kernels (coop_min_l) keeps them, where they fit.
 constexpr long long kRysJkFew = 5000;
 constexpr double rys_jk_item_limit(int la, int lb, int lc, int ld) {
     if (la + lb + lc + ld == 4) return la == 1 ? 5.0 : lb == 2 ? 1.0 : lb == 1 || lc == 2 ? 2.0 : 3.0;
@@ -392,7 +398,7 @@ constexpr double rys_jk_item_limit(int la, int lb, int lc, int ld) {
 }
 inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
-    if (l < (mixed ? kRysMixedL : kRysJkSmallL) || (c->opt.coop_min_l != 0 && l >= c->opt.coop_min_l)) return false;
+    if (l < (mixed ? kRysMixedL : kRysJkSmallL) || asks_coop(c, l, cw.coop_ok)) return false;
     return l >= kRysJkMinL ||
            (cw.quartets <= kRysJkFew && cw.longest_item <= rys_jk_item_limit(cw.la, cw.lb, cw.lc, cw.ld) * cw.heaviest_quartet);
 }
@@ -402,7 +408,7 @@ inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
 // segment in this build is above kGradConcurrentBytes (the scratch bound decides where the table
 // has no entry).
 inline bool on_shared_stream(const hfg_ctx* c, const ClassWork& cw, bool grad, bool mixed) {
-    if (grad ? cw.gcoop || grad_on_rys(c, cw, mixed) : cw.coop || jk_on_rys(c, cw, mixed)) return false;
+    if (grad ? cw.gcoop[mixed] || grad_on_rys(c, cw, mixed) : cw.coop[mixed] || jk_on_rys(c, cw, mixed)) return false;
     if (!grad) return class_spills(cw.la, cw.lb, cw.lc, cw.ld, false);
     const int b = private_segment_bytes(true, mixed, cw.la, cw.lb, cw.lc, cw.ld, c->pure);
     return b < 0 ? class_spills(cw.la, cw.lb, cw.lc, cw.ld, true) : b > kGradConcurrentBytes;

@@ -60,7 +60,7 @@ hipError_t launch_grad_any(hfg_ctx* c, const ClassWork& cw, const GradArgs& b, L
         const RysGradArgs r{b, c->rys, c->pure ? c->d_Dc.p : c->d_D.p, c->d_cart_off.p, c->d_mol_cart.p};
         return launch_rys_grad(cw.la, cw.lb, cw.lc, cw.ld, r, (int)cw.items.size(), sh, st);
     }
-    if (cw.gcoop) return launch_grad_coop(b, cw.gcoop_args, cw.gcoop_lds[mixed], mixed, (int)cw.items.size(), sh, st);
+    if (cw.gcoop[mixed]) return launch_grad_coop(b, cw.gcoop_args, cw.gcoop_lds[mixed], mixed, (int)cw.items.size(), sh, st);
     return launch_grad(cw.la, cw.lb, cw.lc, cw.ld, c->pure, mixed, b, (int)cw.items.size(), sh, st);
 }
 

@@ -1,7 +1,6 @@
 // Run-time dispatch of the adjoint gradient kernels and the fixed-order slab reduction.
 #include "coop_grad.hpp"
 #include "launch_bounds.hpp"
-#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -17,15 +16,13 @@ HFG_FOR_CLASSES(HFG_DECL)
 
 namespace {
 
-// The register kernels: FP64 below L = 4 and for the L = 4 classes with a d shell (the context launches
-// the Rys kernel for the others), mixed below L = 7 (from there it launches the Rys kernel too, or on
-// request the cooperative one, coop_grad.hpp).
+// The register kernels; the context launches the others itself (rys_grad.hpp, coop_grad.hpp).
 template <int A, int B, int C, int D, bool P>
 hipError_t grad_class(const GradArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
     const LaunchShape bs = scratch_safe_shape(A, B, C, D, true, sh, nitems);
-    if constexpr (!grad_uses_coop(A, B, C, D))
+    if constexpr (grad_has_register(A, B, C, D, true))
         if (mixed) return launch_grad_class32<A, B, C, D, P>(a, nitems, bs, s);
-    if constexpr (grad_keeps_register(A, B, C, D))
+    if constexpr (grad_has_register(A, B, C, D, false))
         if (!mixed) return launch_grad_class64<A, B, C, D, P>(a, nitems, bs, s);
     return hipErrorInvalidValue;
 }

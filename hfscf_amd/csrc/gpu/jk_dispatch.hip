@@ -4,7 +4,6 @@
 #include "coop_args.hpp"
 #include "jk_impl.hpp"
 #include "launch_bounds.hpp"
-#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -22,9 +21,9 @@ namespace {
 
 template <int A, int B, int C, int D, bool P>
 hipError_t jk_class(const JkArgs& a, int nitems, LaunchShape sh, int mixed, hipStream_t s) {
-    if constexpr (A + B + C + D < 7)
+    if constexpr (jk_has_register(A, B, C, D, true))
         if (mixed) return launch_jk_class32<A, B, C, D, P>(a, nitems, sh, s);
-    if constexpr (A + B + C + D < kRysJkMinL)
+    if constexpr (jk_has_register(A, B, C, D, false))
         if (!mixed) return launch_jk_class64<A, B, C, D, P>(a, nitems, sh, s);
     return hipErrorInvalidValue;
 }

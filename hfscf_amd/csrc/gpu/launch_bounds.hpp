@@ -3,6 +3,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "rys_layout.hpp"
 
 namespace hfg {
 
@@ -13,6 +14,16 @@ namespace hfg {
 inline size_t class_scratch_bound(int la, int lb, int lc, int ld, bool grad) {
     const int lab = la + lb + (grad ? 1 : 0), lcd = lc + ld + (grad ? 1 : 0), lt = la + lb + lc + ld + (grad ? 1 : 0);
     return sizeof(double) * (size_t)vrr_entries(lab, lcd, lt);
+}
+
+// Whether a class has a per-lane register kernel in a precision; without one it runs the Rys kernel, or on
+// request the cooperative one. Mixed: below L = 7. FP64: J/K below L = 6; the gradient below L = 4 and the
+// L = 4 classes with a d shell.
+constexpr bool jk_has_register(int la, int lb, int lc, int ld, bool mixed) {
+    return la + lb + lc + ld < (mixed ? kRysMixedL : kRysJkMinL);
+}
+constexpr bool grad_has_register(int la, int lb, int lc, int ld, bool mixed) {
+    return mixed ? la + lb + lc + ld < kRysMixedL : grad_keeps_register(la, lb, lc, ld);
 }
 
 // Classes whose register kernels run on the device's shared stream, one at a time. Gradient: every
