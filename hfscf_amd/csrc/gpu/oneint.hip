@@ -140,8 +140,11 @@ struct Overlap1 {
 };
 
 struct PrimPair {
-    double a, b, p, P[3], PA[3], PB[3], K;  // K = exp(-ab/p |AB|^2) c_a c_b
+    double a, b, p, P[3], PA[3], PB[3], r2, K;  // r2 = |AB|^2, K = exp(-ab/p |AB|^2) c_a c_b
 };
+
+// Whether a primitive pair adds nothing; a NaN, or a distance beyond the doubles, shows in the results.
+HFG_INLINE bool vanishes(const PrimPair& pp) { return fabs(pp.K) < kOneTiny && pp.r2 < INFINITY; }
 
 HFG_INLINE PrimPair prim_pair(const OneArgs& g, const OneShell& A, const OneShell& B, int i, int j) {
     const double* ra = g.xyz + 3 * A.atom;
@@ -151,15 +154,15 @@ HFG_INLINE PrimPair prim_pair(const OneArgs& g, const OneShell& A, const OneShel
     pp.b = g.alpha[B.po + j];
     pp.p = pp.a + pp.b;
     const double ip = 1.0 / pp.p;
-    double r2 = 0.0;
+    pp.r2 = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         pp.P[d] = (pp.a * ra[d] + pp.b * rb[d]) * ip;
         pp.PA[d] = pp.P[d] - ra[d];
         pp.PB[d] = pp.P[d] - rb[d];
-        r2 += (ra[d] - rb[d]) * (ra[d] - rb[d]);
+        pp.r2 += (ra[d] - rb[d]) * (ra[d] - rb[d]);
     }
-    pp.K = exp(-pp.a * pp.b * ip * r2) * g.coef[A.po + i] * g.coef[B.po + j];
+    pp.K = exp(-pp.a * pp.b * ip * pp.r2) * g.coef[A.po + i] * g.coef[B.po + j];
     return pp;
 }
 
@@ -178,7 +181,7 @@ __global__ __launch_bounds__(kOneBlock) void oneint_kernel(OneArgs g, const int2
     for (int x = ln; x < nprim * nsl; x += kOneLanes) {
         const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
         const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
-        if (!(fabs(pp.K) >= kOneTiny)) continue;
+        if (vanishes(pp)) continue;
         const double o2p = 0.5 / pp.p;
         if (sl == 0) {
             Overlap1<LA, LB + 2> s[3];
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(kOneBlock) void oneint_grad_kernel(OneArgs g, const
         for (int x = ln; x < nprim * nsl; x += kOneLanes) {
             const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
             const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
-            if (!(fabs(pp.K) >= kOneTiny)) continue;
+            if (vanishes(pp)) continue;
             const double o2p = 0.5 / pp.p, ta = 2.0 * pp.a;
             if (sl == 0) {
                 Overlap1<LA + 1, LB + 2> s[3];
