@@ -150,6 +150,10 @@ HFG_INLINE void hrr_from_vrr(const Vrr<LAB1, LCD1, R>& V, const R* AB, const R* 
 // water / 6-31G* (ss|ss) 576 -> 12 us, (ps|ss) 375 -> 15, (pp|ps) 506 -> 43; its gradient 1.46 -> 0.34 ms.
 constexpr int kGradLanePrims = 512, kGradMinPrims = 8;
 
+// Primitive pair that slice k of a shell pair loads first: one that the pair stores, also when the slice has
+// none or the pair no significant one (np = 0, whose storage still holds the others).
+HFG_HD int first_prim(int k, int np) { return k < np ? k : np > 0 ? np - 1 : 0; }
+
 // Wavefronts per SIMD that the registers of a kernel are held to (1 = no limit). Alone on (H2O)16 /
 // cc-pVDZ in ms, FP64: (ss|ss) 16.7 free, 15.3 at 3; (ps|ss) 20.5, 18.8 at 3; (ps|ps), 4 registers
 // above two wavefronts, 13.6, 11.8 at 2, 32 at 3; (pp|ss) 7.3, 5.8 at 2, 12 at 3; (ds|ss) 3.8, 3.9 at 2;
@@ -259,7 +263,7 @@ grad_kernel(GradArgs a) {
             const double4 a2 = a.pp2[ia];
             const double p = a0.x;
             constexpr bool ahead = lds_boys;  // load the next ket primitive's exponent and centre ahead
-            double4 nb0 = a.pp0[kp.off + min(slk, kp.np - 1) * kp.pstride];
+            double4 nb0 = a.pp0[kp.off + first_prim(slk, kp.np) * kp.pstride];
             for (int jp = slk; jp < kp.np; jp += sk) {
                 const int ib = kp.off + jp * kp.pstride;
                 const double4 b0 = ahead ? nb0 : a.pp0[ib];

@@ -45,3 +45,10 @@ def test_jk_high_l_always(lib, cls):
     for work in ((1, 1, 1), (10 ** 7, 1e5, 1)):
         assert _rys(lib, cls, False, *work)
         assert _rys(lib, cls, True, *work) == (sum(map(int, cls)) >= 7)
+
+
+@pytest.mark.parametrize("np", [0, 1, 2, 9, 81])
+def test_gradient_slices_load_stored_primitives(lib, np):
+    # a slice without primitives of its own loads one of the pair's, which stores one at least
+    for k in range(100):
+        assert lib.grad_first_prim(k, np) == (k if k < np else max(np - 1, 0))
