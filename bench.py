@@ -460,8 +460,8 @@ def main():
     el, kern = time_builds(ctx, Hc, D, args.steps, args.warmup)
     st = ctx.stats()
     classes = ctx.class_stats()  # the last build's class launches, bracketed by HIP events
-    # kernel form of each class's J/K launch: shell-group lists, cooperative, or per-lane register
-    form = {s["cls"]: {-2: "jk_gc", -1: "jk_coop"}.get(s["jk"][1], "jk_kernel") for s in ctx.launch_shapes()}
+    # kernel form of each class's J/K launch: shell-group lists, Rys quadrature, or per-lane register
+    form = {s["cls"]: {-2: "jk_gc", -1: "jk_rys"}.get(s["jk"][1], "jk_kernel") for s in ctx.launch_shapes()}
     for c in classes:
         c["kernel"] = form.get("".join(str(x) for x in c["cls"]), "jk_kernel")
     ctx.close()

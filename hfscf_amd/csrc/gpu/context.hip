@@ -1743,14 +1743,15 @@ int hfg_autotune(hfg_ctx* c, int what) {
 int hfg_launch_shapes(const hfg_ctx* c, int cap, int* la_lb_lc_ld, int* jk_grid, int* jk_block, int* grad_grid,
                       int* grad_block) {
     if (!c) return HFG_ERR_ARG;
-    const int n = (int)c->classes.size(), mixed = c->opt.precision == HFG_MIXED ? 1 : 0;
+    const int n = (int)c->classes.size();
+    const bool mixed = c->opt.precision == HFG_MIXED;
     for (int k = 0; k < n && k < cap; ++k) {
         const ClassWork& cw = c->classes[k];
         if (la_lb_lc_ld) la_lb_lc_ld[k] = cw.la * 1000 + cw.lb * 100 + cw.lc * 10 + cw.ld;
         if (jk_grid) jk_grid[k] = cw.jk_shape.grid;
-        if (jk_block) jk_block[k] = cw.gc ? -2 : cw.coop[mixed] ? -1 : cw.jk_shape.block;
+        if (jk_block) jk_block[k] = cw.gc ? -2 : cw.coop[mixed] || jk_on_rys(c, cw, mixed) ? -1 : cw.jk_shape.block;
         if (grad_grid) grad_grid[k] = cw.grad_shape.grid;
-        if (grad_block) grad_block[k] = cw.gcoop[mixed] ? -1 : cw.grad_shape.block;
+        if (grad_block) grad_block[k] = cw.gcoop[mixed] || grad_on_rys(c, cw, mixed) ? -1 : cw.grad_shape.block;
     }
     return n;
 }

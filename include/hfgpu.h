@@ -224,10 +224,11 @@ int hfg_hessian_2e(hfg_ctx* ctx, const double* D, double* HC, double* HX);
  * workgroup x persistent workgroups) on the density of the most recent build and keeps the
  * fastest per class. what: 1 = J/K, 2 = gradient, 3 = both. */
 int hfg_autotune(hfg_ctx* ctx, int what);
-/* Current launch shape per class (la*1000+lb*100+lc*10+ld, grid, block for J/K and gradient;
- * grid 0 = one workgroup per work item, block 0 = the default, block -1 = the class runs on the
- * cooperative kernel, whose workgroup size is fixed, J/K block -2 = the (ss|ss) class runs on the
- * shell-group kernel, hfg_options.group_shells). Returns the number of classes. */
+/* Current launch shape per class in the context's precision (la*1000+lb*100+lc*10+ld, grid, block for J/K
+ * and gradient; grid 0 = one workgroup per work item, block 0 = the default, block -1 = the class runs
+ * on a kernel of a fixed workgroup size with its tables in LDS: the Rys kernel, or the cooperative one where
+ * hfg_options.coop_min_l or autotuning chose it; J/K block -2 = the class runs on a shell-group kernel,
+ * hfg_options.group_shells). Returns the number of classes. */
 int hfg_launch_shapes(const hfg_ctx* ctx, int cap, int* la_lb_lc_ld, int* jk_grid, int* jk_block, int* grad_grid,
                       int* grad_block);
 

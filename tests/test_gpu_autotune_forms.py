@@ -55,3 +55,18 @@ def test_autotune_mixed_then_fp64(coop_min_l):
     _check(_results(ctx, D), want)
     ctx.set_precision(H.MIXED)
     _check(ctx.build_jk(D), want[:2], (1e-5, 1e-5))
+
+
+def test_launch_shapes_name_the_kernel_form():
+    # block -1: the Rys kernels (FP64 J/K from L = 6 and gradient from L = 4 in a small molecule, mixed from
+    # L = 7) or the cooperative ones that coop_min_l asks for; the others have a block of their own
+    mol = H.Molecule.from_xyz(golden("h2o.xyz"), "cc-pvdz")
+    L = lambda s: sum(int(x) for x in s["cls"])  # noqa: E731
+    ctx = H.GpuContext(mol)
+    for precision, jk_min, grad_min in ((H.FP64, 6, 4), (H.MIXED, 7, 7)):
+        ctx.set_precision(precision)
+        for s in ctx.launch_shapes():
+            if L(s) >= jk_min or L(s) < 4 or precision == H.MIXED:
+                assert (s["jk"][1] == -1) == (L(s) >= jk_min), s
+            assert (s["grad"][1] == -1) == (L(s) >= grad_min), s
+    assert all((s["jk"][1] == -1) == (L(s) >= 5) for s in H.GpuContext(mol, precision=H.MIXED, coop_min_l=5).launch_shapes())
