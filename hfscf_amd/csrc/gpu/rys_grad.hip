@@ -41,14 +41,15 @@ hipError_t launch_rys_jk(int la, int lb, int lc, int ld, const RysJkArgs& a, int
     return hipErrorInvalidValue;
 }
 
-// One thread per Cartesian element; 2 x 2 terms at most, so it moves little more than D and Dc.
+// One thread per Cartesian element; 2 x 2 terms at most, so it moves little more than D and Dc. Molecules on
+// blockIdx.x: a batch may hold more than the 65,536 workgroups of the other dimensions.
 __global__ __launch_bounds__(256) void to_cart_kernel(const double* __restrict__ D, const MolDev* __restrict__ mols,
                                                       const MolCart* __restrict__ mc, const CartTerms* __restrict__ terms,
                                                       double* __restrict__ Dc) {
-    const MolCart m = mc[blockIdx.y];
-    const MolDev md = mols[blockIdx.y];
+    const MolCart m = mc[blockIdx.x];
+    const MolDev md = mols[blockIdx.x];
     const double* Dm = D + md.moff;
-    for (int e = blockIdx.x * 256 + threadIdx.x; e < m.n * m.n; e += gridDim.x * 256) {
+    for (int e = blockIdx.y * 256 + threadIdx.x; e < m.n * m.n; e += gridDim.y * 256) {
         const int i = e / m.n, j = e - i * m.n;
         const CartTerms ti = terms[m.row0 + i], tj = terms[m.row0 + j];
         double v = 0.0;
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256) void to_cart_kernel(const double* __restrict__
 hipError_t launch_to_cart(const double* D, const MolDev* mols, const MolCart* mc, int nmol, int max_ncart,
                           const CartTerms* terms, double* Dc, hipStream_t s) {
     const int grid = std::max(1, std::min(1024, (max_ncart * max_ncart + 255) / 256));
-    hipLaunchKernelGGL(to_cart_kernel, dim3(grid, nmol), dim3(256), 0, s, D, mols, mc, terms, Dc);
+    hipLaunchKernelGGL(to_cart_kernel, dim3(nmol, grid), dim3(256), 0, s, D, mols, mc, terms, Dc);
     return hipGetLastError();
 }
 
