@@ -1869,7 +1869,7 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
         b.queue = c->d_queue.p + k;
         const int n_items = (int)cw.items.size();
         HFG_CHECK(c, launch_zero_ints(b.queue, 1, st));
-        if (jk_on_rys(c, cw, false)) {
+        if (jk_on_rys(c, cw, false, true)) {
             const RysJkArgs ra{b, c->rys, nullptr, c->d_cart_off.p, c->d_mol_cart.p, c->pure ? 1 : 0};
             HFG_CHECK(c, launch_rys_jk(cw.la, cw.lb, cw.lc, cw.ld, ra, n_items, LaunchShape{0, 0}, st));
         } else if (cw.coop[0])

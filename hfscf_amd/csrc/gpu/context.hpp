@@ -390,17 +390,20 @@ inline bool grad_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
 // quartet at a time (per build, program / Rys in ms: (dd|dp), (dp|dd), (dd|dd) of (H2O)8 1.28 / 0.17,
 // 0.49 / 0.08, 0.56 / 0.09, of (H2O)16 1.45 / 0.34, 0.67 / 0.13, 0.56 / 0.09; whole builds 4.35 -> 3.89,
 // 17.9 -> 17.2); below, the FP32 register kernels win ((dp|dp) of (H2O)16 0.62 against 1.06). A context
-// that asks for the program kernels (coop_min_l) keeps them, where they fit.
+// that asks for the program kernels (coop_min_l) keeps them, where they fit. The ERI export (exporting), which
+// digests nothing and flushes no tiles, runs Rys on longer items: vectors in ms at the limit / at 1.5 times it for
+// (pp|pp) and 3 times for the others / at 3 times for all, (H2O)2 6-31G* 0.95 / 0.90 / 0.90, (H2O)4 STO-3G 0.36 / 0.35 /
+// 0.35, (H2O)5 STO-3G 0.46 / 0.46 / 0.53, (H2O)6 STO-3G 0.73 / 0.73 / 0.90.
 constexpr long long kRysJkFew = 5000;
 constexpr double rys_jk_item_limit(int la, int lb, int lc, int ld) {
     if (la + lb + lc + ld == 4) return la == 1 ? 5.0 : lb == 2 ? 1.0 : lb == 1 || lc == 2 ? 2.0 : 3.0;
     return lb == 2 ? 2.0 : lb == 0 ? 6.0 : lc == 2 ? 5.0 : 9.0;
 }
-inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed) {
+inline bool jk_on_rys(const hfg_ctx* c, const ClassWork& cw, bool mixed, bool exporting = false) {
     const int l = cw.la + cw.lb + cw.lc + cw.ld;
     if (l < (mixed ? kRysMixedL : kRysJkSmallL) || asks_coop(c, l, cw.coop_ok)) return false;
-    return l >= kRysJkMinL ||
-           (cw.quartets <= kRysJkFew && cw.longest_item <= rys_jk_item_limit(cw.la, cw.lb, cw.lc, cw.ld) * cw.heaviest_quartet);
+    const double limit = rys_jk_item_limit(cw.la, cw.lb, cw.lc, cw.ld) * (!exporting ? 1.0 : cw.la == 1 ? 1.5 : 3.0);
+    return l >= kRysJkMinL || (cw.quartets <= kRysJkFew && cw.longest_item <= limit * cw.heaviest_quartet);
 }
 
 // Whether a class launch runs on the device's shared stream (one kernel at a time): J/K register
