@@ -784,10 +784,13 @@ int setup_geometry(hfg_ctx* c) {
                 w.C = C;
                 w.D = D;
                 w.mol = m;
-                row_kets.assign(c->bp_cnt[P], 0);
+                // jk_on_rys asks for the longest item of L = 4 and 5 with few shell quartets only
+                const bool by_length = jk_has_rys(cw.la, cw.lb, cw.lc, cw.ld) &&
+                                       cw.la + cw.lb + cw.lc + cw.ld < kRysJkMinL && cw.quartets <= kRysJkFew;
+                if (by_length) row_kets.assign(c->bp_cnt[P], 0);
                 auto push = [&](int r0, int r1, int c0, int c1) {
                     double prims = 0.0;
-                    for (int r = r0; r < r1; ++r)
+                    for (int r = r0; r < r1 && by_length; ++r)
                         prims += c->pairs[c->bp_off[P] + r].np * (cum_np[cum_off[Q] + std::min(row_kets[r], c1)] -
                                                                   cum_np[cum_off[Q] + std::min(row_kets[r], c0)]);
                     cw.longest_item = std::max(cw.longest_item, prims);
@@ -807,8 +810,10 @@ int setup_geometry(hfg_ctx* c) {
                     if (P == Q) cnt = std::min(cnt, i + 1);
                     const double np_i = c->pairs[c->bp_off[P] + i].np;
                     const double kq = np_i * cum_np[cum_off[Q] + cnt];
-                    row_kets[i] = cnt;
-                    cw.heaviest_quartet = std::max(cw.heaviest_quartet, np_i * max_np[cum_off[Q] + cnt]);
+                    if (by_length) {
+                        row_kets[i] = cnt;
+                        cw.heaviest_quartet = std::max(cw.heaviest_quartet, np_i * max_np[cum_off[Q] + cnt]);
+                    }
                     cw.quartets += cnt;
                     cw.flops += kq * fp.per_prim + cnt * fp.per_quartet;
                     cw.grad_flops += kq * gp.per_prim + cnt * gp.per_quartet;

@@ -70,7 +70,8 @@ struct ClassWork {
     std::vector<WorkItem> items;
     size_t dev_off = 0;
     long long quartets = 0;
-    double longest_item = 0, heaviest_quartet = 0;  // primitive quartets of the longest item, the heaviest shell quartet
+    // L = 4 and 5, while quartets <= kRysJkFew: primitive quartets of the longest work item, the heaviest shell quartet
+    double longest_item = 0, heaviest_quartet = 0;
     double flops = 0;
     double grad_flops = 0;
     LaunchShape jk_shape{0, 0};    // persistent workgroups / block of the J/K launch (0 = automatic)
