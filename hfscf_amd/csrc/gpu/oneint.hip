@@ -515,7 +515,7 @@ int one_upload(hfg_ctx* c, hfg::OneArgs& g) {
         return one_fail(c, HFG_ERR_ARG, "one-electron integrals: hfg_set_geometry was given no nuclear charges");
     std::vector<hfg::OneShell> sh(c->nshell);
     for (int s = 0; s < c->nshell; ++s)
-        sh[s] = hfg::OneShell{c->L[s], c->nprim[s], c->prim_off[s], c->atom[s], c->pure ? c->pure_off[s] : c->cart_off[s]};
+        sh[s] = hfg::OneShell{c->L[s], c->nprim[s], c->prim_off[s], c->atom[s]};
     HFG_CHECK(c, hipSetDevice(c->device));
     HFG_CHECK(c, c->d_one_sh.upload(sh, c->stream));
     HFG_CHECK(c, c->d_one_alpha.upload(c->alpha, c->stream));

@@ -7,9 +7,9 @@ struct hfg_ctx;
 namespace hfg {
 
 // A shell for the one-electron kernels: angular momentum, primitive count, offset of its
-// exponents / normalised coefficients, atom, first output-basis function.
+// exponents / normalised coefficients, atom.
 struct OneShell {
-    int L, np, po, atom, ao;
+    int L, np, po, atom;
 };
 
 struct OneArgs {
