@@ -1865,8 +1865,8 @@ int hfg_eri_vector(hfg_ctx* c, double* out, long long count) {
     // streams ((H2O)8 / cc-pVDZ: 16 ms of kernels one after another, 8 ms so)
     HFG_CHECK(c, hipStreamSynchronize(c->stream));
     for (int k : c->class_order[0]) {
-        // the kernel that the class's FP64 J/K builds run (on the per-shell items: a class on the
-        // shell-group lists has them too)
+        // an FP64 J/K kernel of the class (Rys at L = 4 and 5 by the export's own limit), on the per-shell
+        // items, which a class on the shell-group lists has too
         const ClassWork& cw = c->classes[k];
         hipStream_t st = on_shared_stream(c, cw, false, false) ? c->heavy : c->side[std::max(c->class_stream[0][k], 0)];
         JkArgs b = a;

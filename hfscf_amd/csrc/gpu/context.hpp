@@ -116,8 +116,10 @@ struct MolHost {
 // item per 1/1536 of the build's model cost. More items keep more wavefronts in flight and cost more
 // tiles to flush and gather. FP64 builds with the screen at 1, 2, 4 in ms: (H2O)8 4.7, 5.0, 6.0, (H2O)16
 // 25.7, 25.4, 25.9, C12H26 / 6-31G** 4.8, 5.0, 5.5, 64 molecules 9.7, 10.0, 11.2; mixed (H2O)8 3.0, 3.1,
-// 3.8. The gradient has no tiles and wants more: (H2O)8 21.5, 19.5, 18.9, mixed (H2O)16 147, 120, 108.
-// A context without the screen is the gradient's (hfscf's visits every quartet), so the screen decides.
+// 3.8. hfscf's gradient visits every quartet, so a context without the screen is a gradient's; it has no tiles:
+// (H2O)8 21.5, 19.5, 18.9, mixed (H2O)16 147, 120, 108. The gradient of a screened context shares the J/K items; at
+// 1, 4 it takes (H2O)8 18.6, 17.1, mixed (H2O)16 73.9, 70.3, but in 6-31G* (H2O)8 3.1, 3.6, mixed 7.2, 9.0 (items
+// with few shell quartets split each over more lanes, which repeats its density work), so it has no split of its own.
 constexpr double default_work_split(bool screened) { return screened ? 1.0 : 4.0; }
 
 // Cached graph of one J/K build configuration.

@@ -20,10 +20,11 @@
 // once per gradient, so one kernel per class serves both basis types.
 //
 // Bound: LDS reads of step d (six 16-byte reads per component quartet and node against 15 FP64
-// operations) and, in the classes with few components, the load latency of step a. Measured per
-// whole gradient against the kernels before: (H2O)16 / cc-pVDZ 292 -> 171 ms (the (dp|dd), (dd|dp),
+// operations) and, in the classes with few components, the load latency of step a. Measured per whole
+// gradient when every class from L = 4 moved here: (H2O)16 / cc-pVDZ 292 -> 171 ms (the (dp|dd), (dd|dp),
 // (dd|dd) launches 83 ms each -> 4.5, 1.3, 0.1 ms; (dp|pp) 60 -> 28, (dd|pp) 45 -> 4.8, (dp|dp) 50 ->
-// 2.8 ms, each among the other launches), water / 6-31G* 13.7 -> 1.45 ms.
+// 2.8 ms, each among the other launches), water / 6-31G* 13.7 -> 1.45 ms; with the register kernel kept for
+// many (dp|ps), (ds|pp), (ds|ds) and (dd|ss) quartets (grad_on_rys) (H2O)16 148 ms.
 #pragma once
 #include "grad_impl.hpp"
 #include "rys.hpp"

@@ -22,7 +22,9 @@
 // One lane per component quartet forming Hermite convolutions and triple sums of its own lengths
 // (the form before) issued 1.8 scalar instructions per vector instruction and took 1.18 s on (H2O)4 /
 // cc-pVDZ; this form takes 27 ms (water 50 -> 0.76 ms). Bound: the LDS reads of step d in the classes with many
-// components, the load latency and the item's end in the s and p classes.
+// components; in the s and p classes, which take most of the time ((ps|ps) 10 ms, (ss|ss) 7 alone), the load latency
+// and the item's end, two block expansions and 156 global atomics per item, of which every shell quartet has one
+// at least (59 million L2 atomic requests per call there, TCC_ATOMIC).
 #pragma once
 #include "common.hpp"
 #include "oneint.hpp"

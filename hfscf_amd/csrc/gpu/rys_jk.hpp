@@ -14,10 +14,12 @@
 // so a shell quartet whose primitives fall to several wavefronts is digested in parts (the
 // Cartesian diagonal that hfscf takes from its screen is added by the part with the first one).
 //
-// Bound: the latency of a round (three barriers, the loads of step a) at two to three workgroups per
-// CU, about 0.4 ns per primitive quartet over the device; per class against the kernels before in
-// context.hpp (jk_on_rys). Per build: (H2O)8 8.3 -> 6.7 ms, C12H26 / 6-31G** 8.2 -> 5.5 ms, (H2O)16
-// 35.4 -> 29.5 ms.
+// Bound: the latency of a round (four barriers, the loads of step a and its index arithmetic; FP64 is 7 to 17 %
+// of the VALU instructions), about 0.4 ns per primitive quartet over the device. By LDS one workgroup fits a
+// CU for (dd|dd) (134 KB) and (dd|dp) (84 KB), two to four for the other classes. A workgroup walks its work
+// item in series, 2 to 3 us per round of S primitive quartets, which limits the items that L = 4 and 5 run here.
+// Per class against the other kernels in context.hpp (jk_on_rys). Per build, when they replaced the
+// register and program kernels: (H2O)8 8.5 -> 6.4 ms, C12H26 / 6-31G** 8.2 -> 5.5, (H2O)16 34.5 -> 28.7.
 #pragma once
 #include "coop.hpp"
 #include "rys.hpp"

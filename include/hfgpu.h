@@ -65,7 +65,7 @@ typedef struct hfg_options {
     int coop_min_l;       /* 4..7: classes with la+lb+lc+ld >= coop_min_l run on the wavefront-cooperative
                              kernels (one workgroup per quartet, recursion tables in LDS). 0 = the default:
                              the Rys kernels where they are faster (FP64 J/K from L = 6 and gradients from
-                             L = 4, mixed from L = 7, and L = 4 and 5 of small molecules), the per-lane
+                             L = 4, mixed from L = 7, and J/K of L = 4 and 5 in small molecules), the per-lane
                              register kernels elsewhere, where hfg_autotune tries the cooperative form
                              too and keeps what it measures faster for each class. */
     int side_streams;     /* streams the class launches of one build are spread over (1..8, 0 = 6) */
