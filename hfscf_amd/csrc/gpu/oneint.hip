@@ -21,6 +21,7 @@
 // scratch); (H2O)8 / cc-pVDZ gradient terms 0.27 ms (7.9).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -39,8 +40,9 @@ constexpr int kOneLanes = 16;   // lanes per shell pair
 constexpr int kOneBlock = 64;   // threads per workgroup: four shell pairs
 constexpr int kOneLdsAtoms = 1024;  // gradient sums of up to this many nuclei in LDS
 // A primitive pair with exp(-ab/p |AB|^2) c_a c_b below this adds nothing to a double (the integrals
-// are at most a few hundred times it): about half of a water cluster's primitive pairs.
-constexpr double kOneTiny = 1e-40;
+// are at most a few hundred times it): about half of a water cluster's primitive pairs. Not with coordinates
+// beyond kOneFar or infinite, where the other factors overflow and the pair's NaN shows in the results.
+constexpr double kOneTiny = 1e-40, kOneFar = 1e30;
 
 HFG_HD int rsize(int n) { return (n + 1) * (n + 2) * (n + 3) / 6; }
 HFG_HD int ridx(int t, int u, int v) {
@@ -140,11 +142,8 @@ struct Overlap1 {
 };
 
 struct PrimPair {
-    double a, b, p, P[3], PA[3], PB[3], r2, K;  // r2 = |AB|^2, K = exp(-ab/p |AB|^2) c_a c_b
+    double a, b, p, P[3], PA[3], PB[3], K;  // K = exp(-ab/p |AB|^2) c_a c_b
 };
-
-// Whether a primitive pair adds nothing; a NaN, or a distance beyond the doubles, shows in the results.
-HFG_INLINE bool vanishes(const PrimPair& pp) { return fabs(pp.K) < kOneTiny && pp.r2 < INFINITY; }
 
 HFG_INLINE PrimPair prim_pair(const OneArgs& g, const OneShell& A, const OneShell& B, int i, int j) {
     const double* ra = g.xyz + 3 * A.atom;
@@ -154,15 +153,15 @@ HFG_INLINE PrimPair prim_pair(const OneArgs& g, const OneShell& A, const OneShel
     pp.b = g.alpha[B.po + j];
     pp.p = pp.a + pp.b;
     const double ip = 1.0 / pp.p;
-    pp.r2 = 0.0;
+    double r2 = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         pp.P[d] = (pp.a * ra[d] + pp.b * rb[d]) * ip;
         pp.PA[d] = pp.P[d] - ra[d];
         pp.PB[d] = pp.P[d] - rb[d];
-        pp.r2 += (ra[d] - rb[d]) * (ra[d] - rb[d]);
+        r2 += (ra[d] - rb[d]) * (ra[d] - rb[d]);
     }
-    pp.K = exp(-pp.a * pp.b * ip * pp.r2) * g.coef[A.po + i] * g.coef[B.po + j];
+    pp.K = exp(-pp.a * pp.b * ip * r2) * g.coef[A.po + i] * g.coef[B.po + j];
     return pp;
 }
 
@@ -181,7 +180,7 @@ __global__ __launch_bounds__(kOneBlock) void oneint_kernel(OneArgs g, const int2
     for (int x = ln; x < nprim * nsl; x += kOneLanes) {
         const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
         const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
-        if (vanishes(pp)) continue;
+        if (!(fabs(pp.K) >= g.tiny) && pp.K == pp.K) continue;  // a NaN is evaluated
         const double o2p = 0.5 / pp.p;
         if (sl == 0) {
             Overlap1<LA, LB + 2> s[3];
@@ -284,7 +283,7 @@ __global__ __launch_bounds__(kOneBlock) void oneint_grad_kernel(OneArgs g, const
         for (int x = ln; x < nprim * nsl; x += kOneLanes) {
             const int pr = x / nsl, sl = x - pr * nsl, i = pr / B.np;
             const PrimPair pp = prim_pair(g, A, B, i, pr - i * B.np);
-            if (vanishes(pp)) continue;
+            if (!(fabs(pp.K) >= g.tiny) && pp.K == pp.K) continue;  // a NaN is evaluated
             const double o2p = 0.5 / pp.p, ta = 2.0 * pp.a;
             if (sl == 0) {
                 Overlap1<LA + 1, LB + 2> s[3];
@@ -532,6 +531,8 @@ int one_upload(hfg_ctx* c, hfg::OneArgs& g) {
     g.natom = c->natom;
     g.ncart = c->ncart;
     g.cart_off = c->d_cart_off.p;
+    const bool near = std::all_of(c->xyz.begin(), c->xyz.end(), [](double x) { return std::fabs(x) < hfg::kOneFar; });
+    g.tiny = near ? hfg::kOneTiny : 0.0;
     return HFG_OK;
 }
 

@@ -21,6 +21,7 @@ struct OneArgs {
     const double* boys;   // the Boys table
     const int* cart_off;  // shell -> first Cartesian function
     int natom, ncart;
+    double tiny;  // primitive pairs with a prefactor below it are skipped
     double* S;  // ncart x ncart outputs over the Cartesian functions (device)
     double* T;
     double* V;
